@@ -15,7 +15,7 @@
 // Modes (template parameter MODE):
 //   PER_TOKEN  c[m,n] = as[m] · Σ_g ws[n,g]·P_g        (per-token activations)
 //   PER_GROUP  c[m,n] = Σ_g (as[m,g]·ws[n,g])·P_g      (reference matmul_gw;
-//              group 32 on both sides runs on gemm_i8_q8_kernel below)
+//              equal groups of 32, 64 or 128 run on gemm_i8_q8_kernel below)
 //   RAW        c[m,n] = Σ_k a[m,k]·w[n,k]   as int32  (exact)
 //   PARTIALS   p[m,n,g] = P_g                 as int32  (exactness checks)
 //
@@ -322,7 +322,7 @@ __device__ __forceinline__ float glu_apply(float g, float u) {
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int MODE, bool OUT_F16, int MINW = 2,
-          int GLU = GLU_NONE, bool WSF16 = false, int KG = 1>
+          int GLU = GLU_NONE, bool WSF16 = false, int KG = 1, int GB = 1>
 __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
     const int8_t *__restrict__ A, const float *__restrict__ AS, const int8_t *__restrict__ W,
     const float *__restrict__ WS, int ws_stride, void *__restrict__ Cout, int M, int N, int K,
@@ -339,6 +339,11 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
   // SIMD busy on its own, which is what a lone workgroup (a grid of about
   // one tile per CU, or the last round of a larger one) lacks.
   static_assert(KG == 1 || !GROUPED, "K-groups: per-token and raw modes");
+  // GB blocks per weight (and activation) group: with GB 2 and 4 (groups of 64
+  // and 128) a group's blocks accumulate in int32 through the MFMA's C operand
+  // and are folded into f32 once per group.
+  static_assert(GB == 1 || ((GB == 2 || GB == 4) && MODE != MODE_RAW && KG == 1 && GLU == GLU_NONE), "groups");
+  constexpr int GPS = 4 / GB;  // groups per stage
   constexpr bool SCALED = (MODE == MODE_PER_TOKEN) || GROUPED;
   constexpr int CODE_BYTES = (BM + BN) * ROWB;
   constexpr int WS_BYTES = SCALED ? BN * 16 : 0;
@@ -360,9 +365,9 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
   // refilled while the last block's last tile is still to be folded. One row
   // of 32 tiles per wave (TM = 1) keeps one 16-row scale set in registers,
   // shared by the wave's TN column tiles.
-  constexpr int AS_SLOT = GROUPED ? BM * 16 : 0;
-  constexpr int AS_INS = GROUPED ? BM * 4 / 64 : 0;
-  static_assert(!GROUPED || TM == 1, "per-group mode: one row of 32x32 tiles per wave");
+  constexpr int AS_SLOT = GROUPED ? BM * 4 * GPS : 0;
+  constexpr int AS_INS = GROUPED ? BM * GPS / 64 : 0;
+  static_assert(!GROUPED || GB > 1 || TM == 1, "per-block groups: one row of 32x32 tiles per wave");
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float *s_as = (float *)(smem + KG * STAGES * STAGE_BYTES);  // [BM] per-token activation scales
@@ -394,7 +399,7 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
   const uint32_t voff_even = r8 * K + ((p8 ^ (r8 >> 1)) << 4);
   const uint32_t voff_odd = r8 * K + ((p8 ^ (4 + (r8 >> 1))) << 4);
   const uint32_t voff_ws = lane * ws_stride * 4;
-  // per-group scale copy c: float f = 64c + lane of the slot = (block f / BM, row f % BM)
+  // per-group scale copy c: float f = 64c + lane of the slot = (group f / BM, row f % BM)
   const rsrc_t ras = make_rsrc(GROUPED ? AS + (size_t)m0 * as_stride : AS,
                                GROUPED ? (int64_t)(M - m0) * as_stride * 4 : 0);
   auto as_voff = [&](int c) -> uint32_t {
@@ -432,7 +437,7 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
       for (int c = 0; c < AS_INS; ++c)
         if (wave == NW - 1 - c % NW)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(ras, LDS_PTR(ab + c * 256), 4, as_voff(c),
-                                                   (uint32_t)(kt * 16), 0, 0);
+                                                   (uint32_t)(kt * 4 * GPS), 0, 0);
     }
   };
   // Make stage kt visible to every wave. Copies return in issue order, so
@@ -472,10 +477,11 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
   floatx4 as_pend[4];  // per-group scales of the block whose tile is folded next
 #pragma unroll
   for (int q = 0; q < 4; ++q) as_pend[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto load_as = [&](floatx4(&dst)[4], int g) {
-    const uint8_t *ab = s_asg + ((g >> 2) % (STAGES + 1)) * AS_SLOT + (g & 3) * BM * 4 + asg_off;
+  // the scales of tile row i for the group that holds block g
+  auto load_as = [&](floatx4(&dst)[4], int g, int i = 0) {
+    const uint8_t *ab = s_asg + ((g >> 2) % (STAGES + 1)) * AS_SLOT + (g & 3) / GB * BM * 4 + asg_off;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dst[q] = *(const floatx4 *)(ab + q * 32);
+    for (int q = 0; q < 4; ++q) dst[q] = *(const floatx4 *)(ab + i * 128 + q * 32);
   };
 
   intx4 af[2][TM], bf[2][TN];
@@ -534,6 +540,27 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
 #pragma unroll
   for (int r = 0; r < 16; ++r) ires[0][r] = ires[1][r] = 0;
   float dpend = 0.f;  // scale of the pending tile (the last tile of the previous block)
+  // GB > 1: the column scales of the group whose int32 sums (iacc) wait to be
+  // folded. The group's fold runs tile by tile between the MFMAs of the next
+  // group's first block, each of which then starts its tile from zero.
+  float dgrp[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) dgrp[j] = 0.f;
+  auto fold_group = [&](auto i_c, auto j_c, int g) {  // g: a block of the group
+    constexpr int I = decltype(i_c)::value, J = decltype(j_c)::value;
+    if constexpr (GROUPED && J == 0) load_as(as_pend, g, I);
+    static_for<4>([&](auto q_c) {
+      constexpr int Q = decltype(q_c)::value;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 4 * Q + e;
+        const float sc = GROUPED ? as_pend[Q][e] * dgrp[J] : dgrp[J];
+        facc[I][J][r] = __builtin_fmaf((float)iacc[I][J][r], sc, facc[I][J][r]);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // four elements' temporaries at a time
+    });
+  };
+
   // Per-group mode with fp16 weight scales (WSF16): each MFMA starts from the
   // int32 bits of 1.5·2^23 (GBIAS_BITS), so its result read as a float is
   // exactly 1.5·2^23 + P_g (|P_g| < 2^19); fma(F, d, -1.5·2^23·d) is then
@@ -591,6 +618,22 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
 #pragma unroll
         for (int j = 0; j < TN; ++j)
           iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[CUR][i], bf[CUR][j], iacc[i][j], 0, 0, 0);
+    } else if constexpr (GB > 1) {
+      load_frags(ic<NXT>{}, ic<NS>{}, ic<NB>{});
+      static_for<TM * TN>([&](auto uc) {
+        constexpr int I = decltype(uc)::value / TN, J = decltype(uc)::value % TN;
+        if constexpr (B % GB == 0) {
+          if (B != 0 || g > 0) fold_group(ic<I>{}, ic<J>{}, g - 1);
+          __builtin_amdgcn_sched_barrier(0);
+          iacc[I][J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[CUR][I], bf[CUR][J], intx16{}, 0, 0, 0);
+        } else {
+          iacc[I][J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[CUR][I], bf[CUR][J], iacc[I][J], 0, 0, 0);
+        }
+      });
+      if constexpr (B % GB == GB - 1) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) dgrp[j] = dsc[CUR][j];
+      }
     } else {
       // Tile 0 of this block first: its wait covers only the fragments read
       // in the previous step. Then the next block's fragments are read from
@@ -633,7 +676,9 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
     if constexpr (STAGES > 1) stage(ic<1>{});
     if constexpr (STAGES > 2) stage(ic<2>{});
   }
-  if constexpr (SCALED) {
+  if constexpr (GB > 1) {
+    static_for<TM * TN>([&](auto uc) { fold_group(ic<decltype(uc)::value / TN>{}, ic<decltype(uc)::value % TN>{}, NBLK - 1); });
+  } else if constexpr (SCALED) {
     // The last block's last tile sits in set ((NBLK-1)·T + T-1) & 1.
     if (((NBLK * T - 1) & 1) != 0)
       fold(ic<1>{}, ic<TM - 1>{}, ic<TN - 1>{}, dpend, as_pend);
@@ -737,14 +782,14 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int MODE, bool OUT_F16, int MINW = 2,
-          int GLU = GLU_NONE, bool WSF16 = false, int KG = 1>
+          int GLU = GLU_NONE, bool WSF16 = false, int KG = 1, int GB = 1>
 static hipError_t launch_q8(const I8GemmArgs &g, hipStream_t st) {
   constexpr bool SCALED = MODE == MODE_PER_TOKEN || MODE == MODE_PER_GROUP;
   constexpr int smem = KG * STAGES * ((BM + BN) * 128 + (SCALED ? BN * 16 : 0)) +
-                       (MODE == MODE_PER_GROUP ? (STAGES + 1) * BM * 16 : BM * 4);
+                       (MODE == MODE_PER_GROUP ? (STAGES + 1) * BM * (16 / GB) : BM * 4);
   static_assert(smem <= 160 * 1024, "LDS");
   if (KG > 1 && g.K % (128 * KG) != 0) return hipErrorInvalidValue;
-  auto kern = gemm_i8_q8_kernel<BM, BN, WM, WN, STAGES, MODE, OUT_F16, MINW, GLU, WSF16, KG>;
+  auto kern = gemm_i8_q8_kernel<BM, BN, WM, WN, STAGES, MODE, OUT_F16, MINW, GLU, WSF16, KG, GB>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void *)kern,
@@ -885,6 +930,27 @@ static hipError_t launch_q8g(int c, const I8GemmArgs &g, hipStream_t st) {
   return launch_q8<64, 128, 2, 4, 2, MODE_PER_GROUP, OUT_F16, 4, GLU_NONE, WSF16>(g, st);
 }
 
+// Groups of 64 and 128 on the pipelined kernel: MFMA-bound like the raw
+// product, with one fold (convert, scale, FMA) per 64 or 128 K-values instead
+// of one per 32. 128x64 tiles on 4 waves of 64x32 (two workgroups per CU) while
+// they cover the CUs at least once, 64x64 below that. MI355X, the call with
+// its quantizer: 2777x1024->3072 in groups of 128 / 64 took 91.0 / 87 us on
+// gemm_i8_kernel, 30.3 / 37.0 us here (the GEMM 27.1); 128x128 tiles on 8 waves are 34.1 / 41.0
+// and on 4 waves spill (50 / 80 us).
+template <int MODE, bool OUT_F16, int GB>
+static hipError_t launch_q8_groups(const I8GemmArgs &g, hipStream_t st) {
+  const long t128 = ((g.M + 127) / 128) * (long)((g.N + 127) / 128);
+  if (2 * t128 >= g.num_cus)
+    return launch_q8<128, 64, 2, 2, 3, MODE, OUT_F16, 2, GLU_NONE, false, 1, GB>(g, st);
+  return launch_q8<64, 64, 2, 2, 3, MODE, OUT_F16, 2, GLU_NONE, false, 1, GB>(g, st);
+}
+template <int MODE>
+static hipError_t dispatch_groups(const I8GemmArgs &g, hipStream_t st) {
+  if (g.gb == 2)
+    return g.out_f16 ? launch_q8_groups<MODE, true, 2>(g, st) : launch_q8_groups<MODE, false, 2>(g, st);
+  return g.out_f16 ? launch_q8_groups<MODE, true, 4>(g, st) : launch_q8_groups<MODE, false, 4>(g, st);
+}
+
 hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st) {
   switch (g.mode) {
     case I8_PER_TOKEN:
@@ -897,6 +963,7 @@ hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st) {
         return g.out_f16 ? launch_q8_cfg<true>(g, st) : launch_q8_cfg<false>(g, st);
       }
       if (g.glu != 0) return hipErrorInvalidValue;
+      if (g.gb == 2 || g.gb == 4) return dispatch_groups<MODE_PER_TOKEN>(g, st);
       return dispatch_scaled<MODE_PER_TOKEN>(g, st);
     case I8_PER_GROUP:
       // Group-32 activations against a group-32 weight: pipelined kernel
@@ -908,6 +975,7 @@ hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st) {
         return g.ws_f16 ? (g.out_f16 ? launch_q8g<true, true>(c, g, st) : launch_q8g<false, true>(c, g, st))
                         : (g.out_f16 ? launch_q8g<true, false>(c, g, st) : launch_q8g<false, false>(c, g, st));
       }
+      if ((g.gb == 2 || g.gb == 4) && g.a_gb == g.gb) return dispatch_groups<MODE_PER_GROUP>(g, st);
       return dispatch_scaled<MODE_PER_GROUP>(g, st);
     case I8_RAW: {
       // Two K-groups of waves per workgroup where the grid leaves a CU with
