@@ -39,27 +39,13 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "glu.hpp"
 #include "kernels.hpp"
 
 namespace {
 constexpr int KS = 64;    // K values per stage
 constexpr int ROWB = 128;  // bytes per LDS row of one stage
 }  // namespace
-
-// MLP glue of a gate|up product, in f32 in the reference's operation order
-// with no FMA contraction (host.rs:12-39): 1 silu(g)·u, 2 gelu_tanh(g)·u.
-template <int GLU>
-__device__ __forceinline__ float f16_glu(float g, float u) {
-#pragma clang fp contract(off)
-  if constexpr (GLU == 1) {
-    const float sigmoid = 1.0f / (1.0f + expf(-g));
-    return g * sigmoid * u;
-  } else {
-    constexpr float k = (float)(1.12837916709551257390 * 0.70710678118654752440);  // sqrt(2/pi)
-    const float inner = (g + g * g * g * 0.044715f) * k;
-    return ((g * (tanhf(inner) + 1.0f)) * 0.5f) * u;
-  }
-}
 
 // GLU = 0: C [M, N] fp16. GLU = 1 / 2: B holds gate and up rows interleaved
 // per 16 (rows 32t..32t+15 gate rows 16t.., rows 32t+16.. the matching up
@@ -282,7 +268,7 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = (float)(f16)acc[i][j][e], u = (float)(f16)acc[i][j + 1][e];
-          y[e] = f16_glu<GLU>(g, u);
+          y[e] = glu_apply<GLU>(g, u);
         }
         if constexpr (OUT_F16) {
           f16 *crow_p = (f16 *)Cv + (size_t)m * n_out;

@@ -33,6 +33,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "glu.hpp"
 #include "kernels.hpp"
 
 enum { MODE_PER_TOKEN = 0, MODE_PER_GROUP = 1, MODE_RAW = 2, MODE_PARTIALS = 3 };
@@ -301,25 +302,10 @@ static hipError_t launch_i8(const I8GemmArgs &g, hipStream_t st) {
 // scaled mode is VALU-bound at 1/4 of the int8 MFMA rate.
 // ---------------------------------------------------------------------------
 
-// MLP glue applied to column pairs in the epilogue (GLU_SILU: silu(g)·u,
-// GLU_GELU: gelu_tanh(g)·u, the formulas of host.rs:12-39 in f32 without FMA
-// contraction). The weight rows come interleaved in 16-row groups, gate rows
+// MLP glue applied to column pairs in the epilogue (glu.hpp). The weight rows come interleaved in 16-row groups, gate rows
 // 16q..16q+15 at 32q..32q+15 and the matching up rows at 32q+16..32q+31, so
 // in a 32-column MFMA tile lane l (l%32 < 16) holds a gate value and lane
 // l+16 the up value of the same output (row m, column 16q + l%32).
-enum { GLU_NONE = 0, GLU_SILU = 1, GLU_GELU = 2 };
-template <int GLU>
-__device__ __forceinline__ float glu_apply(float g, float u) {
-#pragma clang fp contract(off)
-  if constexpr (GLU == GLU_SILU) {
-    const float sigmoid = 1.0f / (1.0f + expf(-g));
-    return g * sigmoid * u;
-  } else {
-    constexpr float k = (float)(1.12837916709551257390 * 0.70710678118654752440);  // sqrt(2/pi)
-    const float inner = (g + g * g * g * 0.044715f) * k;
-    return ((g * (tanhf(inner) + 1.0f)) * 0.5f) * u;
-  }
-}
 
 template <int BM, int BN, int WM, int WN, int STAGES, int MODE, bool OUT_F16, int MINW = 2,
           int GLU = GLU_NONE, bool WSF16 = false, int KG = 1, int GB = 1>
@@ -952,6 +938,7 @@ static hipError_t dispatch_groups(const I8GemmArgs &g, hipStream_t st) {
 }
 
 hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st) {
+  if (rk_gemm_i8_skinny(g)) return rk_launch_gemm_i8_skinny(g, st);
   switch (g.mode) {
     case I8_PER_TOKEN:
       // One scale per 32-value block (GGUF Q8_0 / group 32): pipelined kernel.

@@ -63,6 +63,14 @@ struct I8GemmArgs {
   int n_out = 0;
 };
 hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st);
+// GEMMs with few output tiles (skinny.hip): whether a launch goes there, and
+// the launches. fp16: C [M, N] fp16, or with glu the gate|up forms above; n is
+// N, or n_out of a gate|up product.
+bool rk_gemm_i8_skinny(const I8GemmArgs &g);
+hipError_t rk_launch_gemm_i8_skinny(const I8GemmArgs &g, hipStream_t st);
+bool rk_gemm_f16_skinny(int M, int n, bool glu, int num_cus);
+hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
+                                     bool out_f16, int num_cus, hipStream_t st);
 
 // Element-wise conversions.
 hipError_t rk_launch_f32_to_f16(const float *x, void *y, int64_t n, hipStream_t st);

@@ -1,0 +1,341 @@
+// GEMMs with few output tiles (decode steps, search queries, short batches) on
+// gfx950: int8 with one scale per weight group, and fp16.
+//
+// What bounds these is latency, not bytes: the tiled kernels walk K stage by
+// stage in each workgroup, with a barrier and an LDS round trip per stage, on
+// a grid of a few dozen workgroups. Here a workgroup of 8 waves takes one
+// 32x32 (int8) or 16x16 to 32x16 (fp16; gate|up 32 weight rows) output tile
+// and the waves split K: wave w takes stages w, w + 8, ..., loads the MFMA
+// operands of its stages straight from memory into registers (no other wave of
+// the workgroup reads the same bytes, so LDS would only add a trip; the loads
+// of a stage and of the wave's next one are in flight together), and the
+// partial sums meet once, in LDS, added in wave order. The order of the sums
+// depends on K alone, so a fused gate|up product equals plain products that also
+// run here bit for bit. Measured on MI355X (us per call, tiled kernel -> here):
+//   int8 per token   12 rows, 1024->3072 8.7 -> 4.0;  3072->1024 20.0 -> 7.2;
+//                    256 rows, 3072->1024 20.5 -> 8.8
+//   int8 group 32    16 rows, 1024->3072 11.1 -> 4.4; 256 rows, 3072->1024 28.5 -> 11.4
+//   fp16             1 row, 1024->3072 5.4 -> 3.4;    64 rows, 3072->1024 11.6 -> 7.2
+// 16 waves per workgroup gain 0.4 us on K = 3072 and lose as much on K = 1024;
+// int8 workgroups of 64 rows (half the weight reads) are 0.8 to 3.4 us slower.
+#include "common.hpp"
+#include "glu.hpp"
+#include "kernels.hpp"
+
+namespace {
+constexpr int SNW = 8;  // waves per workgroup, the K split
+
+__device__ __forceinline__ float glu_any(int glu, float g, float u) {
+  return glu == GLU_SILU ? glu_apply<GLU_SILU>(g, u) : glu_apply<GLU_GELU>(g, u);
+}
+}  // namespace
+
+// int8: C[m, n] = Σ_g (as[m, g]·)ws[n, g]·P_g (times as[m] per token), P_g the
+// exact int32 product of a group of GB 32-value blocks. A stage is 128 K-values
+// (4 blocks, one v_mfma_i32_32x32x32_i8 each).
+template <bool GROUPED, int GB>
+__global__ __launch_bounds__(SNW * 64, 2) void skinny_i8_kernel(
+    const int8_t *__restrict__ A, const float *__restrict__ AS, int as_stride, const int8_t *__restrict__ W,
+    const float *__restrict__ WS, int ws_stride, void *__restrict__ C, int M, int N, int K, int out_f16,
+    int glu, int n_out) {
+  constexpr int GPS = 4 / GB;  // groups per stage
+  __shared__ __attribute__((aligned(16))) float red[SNW * 1024];  // [wave][16][64]
+
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fcol = lane & 31, fh = lane >> 5;
+  const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
+  const int rows = min(M - m0, 32), cols = min(N - n0, 32);
+  const int KT = (K + 127) / 128, KB = K / 32;
+
+  // Rows past M and N read as zeros (offsets past the end of the buffers).
+  const rsrc_t ra = make_rsrc(A + (size_t)m0 * K, (int64_t)rows * K);
+  const rsrc_t rw = make_rsrc(W + (size_t)n0 * K, (int64_t)cols * K);
+  const rsrc_t rs = make_rsrc(WS + (size_t)n0 * ws_stride, (int64_t)cols * ws_stride * 4);
+  const rsrc_t ras = make_rsrc(AS + (size_t)m0 * as_stride, (int64_t)rows * as_stride * 4);
+  const uint32_t v_row = (uint32_t)(fcol * K + fh * 16);
+  const uint32_t v_ws = (uint32_t)(fcol * ws_stride * 4);
+
+  struct Stage {
+    intx4 a[4], w[4];
+    floatx4 ws;
+    float as[GPS];
+  } st[2];
+  auto load = [&](Stage &s, int kt) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) s.w[b] = __builtin_amdgcn_raw_buffer_load_b128(rw, v_row + 32 * b, kt * 128, 0);
+    s.ws = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, v_ws, kt * 16, 0));
+#pragma unroll
+    for (int b = 0; b < 4; ++b) s.a[b] = __builtin_amdgcn_raw_buffer_load_b128(ra, v_row + 32 * b, kt * 128, 0);
+    if constexpr (GROUPED) {
+#pragma unroll
+      for (int g = 0; g < GPS; ++g)
+        s.as[g] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(ras, (uint32_t)((fcol * as_stride + g) * 4), kt * GPS * 4, 0));
+    }
+  };
+
+  floatx16 facc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) facc[r] = 0.f;
+  // The wave's part of `red` first holds the stage's activation scales,
+  // [group][row]: lane `row` has them, every lane needs 16 rows'. A wave's LDS
+  // accesses run in order, so nothing waits between them.
+  float *s_as = red + wave * 1024;
+  auto stage = [&](const Stage &s, int kt) {
+    if constexpr (GROUPED) {
+      asm volatile("" ::: "memory");
+      if (fh == 0) {
+#pragma unroll
+        for (int g = 0; g < GPS; ++g) s_as[g * 32 + fcol] = s.as[g];
+      }
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int g = 0; g < GPS; ++g) {
+      if (kt * 4 + g * GB >= KB) break;  // wave-uniform: K ends inside the stage
+      const float d = s.ws[g * GB];
+      intx16 p = {};
+#pragma unroll
+      for (int b = 0; b < GB; ++b)
+        p = __builtin_amdgcn_mfma_i32_32x32x32_i8(s.a[g * GB + b], s.w[g * GB + b], p, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        floatx4 as4 = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (GROUPED) as4 = *(const floatx4 *)(s_as + g * 32 + q * 8 + fh * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float sc = GROUPED ? as4[e] * d : d;
+          facc[4 * q + e] = __builtin_fmaf((float)p[4 * q + e], sc, facc[4 * q + e]);
+        }
+      }
+    }
+  };
+
+  if (wave < KT) load(st[0], wave);
+  for (int kt = wave; kt < KT; kt += 2 * SNW) {
+    if (kt + SNW < KT) load(st[1], kt + SNW);
+    stage(st[0], kt);
+    if (kt + SNW < KT) {
+      if (kt + 2 * SNW < KT) load(st[0], kt + 2 * SNW);
+      stage(st[1], kt + SNW);
+    }
+  }
+
+#pragma unroll
+  for (int r = 0; r < 16; ++r) red[wave * 1024 + r * 64 + lane] = facc[r];
+  __syncthreads();
+  // Element e = r·64 + lane: row 8·(r/4) + 4·(lane/32) + r%4,
+  // column lane%32 (gate|up: columns 0..15 gate, 16..31 up).
+  auto value = [&](int e, int m) {
+    float v = red[e];
+#pragma unroll
+    for (int w = 1; w < SNW; ++w) v += red[w * 1024 + e];
+    return GROUPED ? v : AS[(size_t)m * as_stride] * v;
+  };
+  auto row_of = [&](int e) { return m0 + (e >> 8) * 8 + ((e >> 5) & 1) * 4 + ((e >> 6) & 3); };
+  if (glu != GLU_NONE) {
+    {
+      const int p = threadIdx.x;  // 512 gate|up pairs
+      const int e = (p >> 4) * 32 + (p & 15);
+      const int m = row_of(e), oc = n0 / 2 + (p & 15);
+      if (m < M && oc < n_out) {
+        const float y = glu_any(glu, value(e, m), value(e + 16, m));
+        if (out_f16)
+          ((f16 *)C)[(size_t)m * n_out + oc] = (f16)y;
+        else
+          ((float *)C)[(size_t)m * n_out + oc] = y;
+      }
+    }
+    return;
+  }
+  for (int e = threadIdx.x; e < 1024; e += SNW * 64) {
+    const int m = row_of(e), n = n0 + (e & 31);
+    if (m < M && n < N) {
+      const float y = value(e, m);
+      if (out_f16)
+        ((f16 *)C)[(size_t)m * N + n] = (f16)y;
+      else
+        ((float *)C)[(size_t)m * N + n] = y;
+    }
+  }
+}
+
+template <bool GROUPED, int GB>
+static hipError_t launch_skinny_i8(const I8GemmArgs &g, hipStream_t st) {
+  hipLaunchKernelGGL((skinny_i8_kernel<GROUPED, GB>), dim3((g.N + 31) / 32, (g.M + 31) / 32), dim3(SNW * 64), 0, st,
+                     g.A, g.AS, g.as_stride, g.W, g.WS, g.ws_stride, g.C, g.M, g.N, g.K, (int)g.out_f16, g.glu,
+                     g.glu ? g.n_out : g.N);
+  return hipGetLastError();
+}
+
+// By the number of 32x32 output tiles (of one product of a gate|up pair, so
+// that the fused and the plain form take the same kernel) against the CUs:
+// past about two rounds of workgroups the weights and activations re-read by
+// every tile cost more than the tiled kernel's serial stages. MI355X, 256 CUs,
+// tiled -> here: per token 1024->3072 480 tiles 9.3 -> 6.7 us, 576 tiles 9.2 ->
+// 9.1; 1152->4304 405 tiles 9.9 -> 6.8, 540 tiles 10.0 -> 9.5. Groups of 64 and
+// 128 fold less and their tiled kernel is faster: 1024->3072 192 tiles 5.9 ->
+// 4.6 us, 288 tiles 6.0 -> 6.8. A tile forced by RK_Q8_TILE / RK_Q8G_TILE
+// keeps the tiled kernel; RK_SKINNY=0 turns these kernels off.
+bool rk_gemm_i8_skinny(const I8GemmArgs &g) {
+  const bool token = g.mode == I8_PER_TOKEN, group = g.mode == I8_PER_GROUP && g.a_gb == g.gb;
+  if (!(token || group) || (g.gb != 1 && g.gb != 2 && g.gb != 4)) return false;
+  if (rk_knob("RK_SKINNY", 1) == 0 || rk_knob(token ? "RK_Q8_TILE" : "RK_Q8G_TILE", -1) >= 0) return false;
+  const int64_t n = g.glu ? g.n_out : g.N;
+  const int64_t tiles = ((g.M + 31) / 32) * ((n + 31) / 32);
+  return g.gb == 1 ? 2 * tiles <= 3 * (int64_t)g.num_cus : tiles <= g.num_cus;
+}
+
+hipError_t rk_launch_gemm_i8_skinny(const I8GemmArgs &g, hipStream_t st) {
+  if (g.mode == I8_PER_TOKEN) {
+    if (g.gb == 1) return launch_skinny_i8<false, 1>(g, st);
+    if (g.gb == 2) return launch_skinny_i8<false, 2>(g, st);
+    if (g.gb == 4) return launch_skinny_i8<false, 4>(g, st);
+  } else if (g.mode == I8_PER_GROUP) {
+    if (g.gb == 1) return launch_skinny_i8<true, 1>(g, st);
+    if (g.gb == 2) return launch_skinny_i8<true, 2>(g, st);
+    if (g.gb == 4) return launch_skinny_i8<true, 4>(g, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+// fp16: a stage is 64 K-values (two v_mfma_f32_16x16x32_f16 steps), TM 16-row
+// tiles, TN 16-row weight tiles (2: gate and up of 16 outputs). The MFMA forms
+// Cᵀ tiles, so a lane holds 4 consecutive columns of one row.
+template <int TM, int TN>
+__global__ __launch_bounds__(SNW * 64, 2) void skinny_f16_kernel(const f16 *__restrict__ A, const f16 *__restrict__ B,
+                                                                 void *__restrict__ C, int M, int N, int K,
+                                                                 int out_f16, int glu, int n_out) {
+  constexpr int T = TM * TN;
+  __shared__ __attribute__((aligned(16))) float red[SNW * T * 256];  // [wave][tile][lane][4]
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * (16 * TN), m0 = blockIdx.y * (16 * TM);
+  const int rows = min(M - m0, 16 * TM), cols = min(N - n0, 16 * TN);
+  const int KT = (K + 63) / 64;
+
+  const rsrc_t ra = make_rsrc(A + (size_t)m0 * K, (int64_t)rows * K * 2);
+  const rsrc_t rb = make_rsrc(B + (size_t)n0 * K, (int64_t)cols * K * 2);
+  const uint32_t v_row = (uint32_t)((l16 * K + lg * 8) * 2);
+  const bool ktail = (K % 64) != 0;
+
+  struct Stage {
+    half8 a[2][TM], b[2][TN];
+  } st[2];
+  auto load = [&](Stage &s, int kt) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      // chunks past K read as zeros
+      const bool past = ktail && kt * 64 + u * 32 + lg * 8 >= K;
+      const uint32_t v = past ? OOB_OFFSET : v_row + u * 64;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        s.b[u][j] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(rb, past ? OOB_OFFSET : v + j * 32 * K, kt * 128, 0));
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        s.a[u][i] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(ra, past ? OOB_OFFSET : v + i * 32 * K, kt * 128, 0));
+    }
+  };
+  floatx4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto stage = [&](const Stage &s) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(s.b[u][j], s.a[u][i], acc[i][j], 0, 0, 0);
+  };
+  if (wave < KT) load(st[0], wave);
+  for (int kt = wave; kt < KT; kt += 2 * SNW) {
+    if (kt + SNW < KT) load(st[1], kt + SNW);
+    stage(st[0]);
+    if (kt + SNW < KT) {
+      if (kt + 2 * SNW < KT) load(st[0], kt + 2 * SNW);
+      stage(st[1]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) *(floatx4 *)(red + ((wave * T + i * TN + j) * 64 + lane) * 4) = acc[i][j];
+  __syncthreads();
+  auto value = [&](int t, int e) {  // element e of tile t: row (e/4)%16, column 4·(e/64) + e%4
+    float v = red[t * 256 + e];
+#pragma unroll
+    for (int w = 1; w < SNW; ++w) v += red[(w * T + t) * 256 + e];
+    return v;
+  };
+  if (glu != GLU_NONE) {
+    for (int x = threadIdx.x; x < TM * 256; x += SNW * 64) {
+      const int i = x >> 8, c = x & 15, r = (x >> 4) & 15;  // columns fastest: coalesced stores
+      const int e = (c >> 2) * 64 + r * 4 + (c & 3);
+      const int m = m0 + i * 16 + r, oc = n0 / 2 + c;
+      if (m < M && oc < n_out) {
+        const float g = (float)(f16)value(i * TN, e), u = (float)(f16)value(i * TN + TN - 1, e);
+        const float y = glu_any(glu, g, u);
+        if (out_f16)
+          ((f16 *)C)[(size_t)m * n_out + oc] = (f16)y;
+        else
+          ((float *)C)[(size_t)m * n_out + oc] = y;
+      }
+    }
+    return;
+  }
+  for (int x = threadIdx.x; x < T * 256; x += SNW * 64) {
+    const int t = x >> 8, c = x & 15, r = (x >> 4) & 15;
+    const int m = m0 + (t / TN) * 16 + r, n = n0 + (t % TN) * 16 + c;
+    if (m < M && n < N) ((f16 *)C)[(size_t)m * N + n] = (f16)value(t, (c >> 2) * 64 + r * 4 + (c & 3));
+  }
+}
+
+template <int TM, int TN>
+static hipError_t launch_skinny_f16(const void *A, const void *B, void *C, int M, int N, int K, bool out_f16, int glu,
+                                    int n_out, hipStream_t st) {
+  hipLaunchKernelGGL((skinny_f16_kernel<TM, TN>), dim3((N + 16 * TN - 1) / (16 * TN), (M + 16 * TM - 1) / (16 * TM)),
+                     dim3(SNW * 64), 0, st, (const f16 *)A, (const f16 *)B, C, M, N, K, (int)out_f16, glu, n_out);
+  return hipGetLastError();
+}
+
+// The smallest tile (1x1, 2x1 or 1x2 of 16x16) that one round of workgroups
+// covers, none if that takes larger ones: 32x32 tiles lose to the tiled kernel
+// (1152->4304, 32 rows: 6.1 us tiled, 6.4 us on 32x32). MI355X, tiled -> here:
+// 1024->4096 32 rows (2x1) 5.7 -> 4.8 us; 1152->4304 16 rows (1x2) 5.9 -> 5.1;
+// 3072->1024 64 rows (1x1) 11.6 -> 7.2, 128 rows (2x1) 11.7 -> 10.0. A gate|up
+// product needs a gate and an up tile per workgroup (1x2): 1024->2x3072 12 rows
+// 5.5 -> 4.6 us, 3072->2x1024 64 rows 11.5 -> 10.1; past one round it loses
+// (1152->2x4304 12 rows, 269 workgroups: 6.0 -> 7.5), and 32x32 tiles lose there
+// too (3072->2x1024 128 rows 11.6 -> 13.0). n: the outputs of one product of a gate|up pair. A tile or split
+// forced by RK_F16_TILE / RK_F16_KSPLIT keeps the tiled kernel.
+static int f16_skinny_tile(int M, int n, bool glu, int num_cus) {
+  if (M > 128) return 0;
+  const int64_t m16 = (M + 15) / 16, m32 = (M + 31) / 32, n16 = (n + 15) / 16, n32 = (n + 31) / 32;
+  if (glu) return m16 * n16 <= num_cus ? 12 : 0;
+  if (m16 * n16 <= num_cus) return 11;
+  if (m32 * n16 <= num_cus) return 21;
+  return m16 * n32 <= num_cus ? 12 : 0;
+}
+
+bool rk_gemm_f16_skinny(int M, int n, bool glu, int num_cus) {
+  if (rk_knob("RK_SKINNY", 1) == 0 || rk_knob("RK_F16_TILE", -1) >= 0 || rk_knob("RK_F16_KSPLIT", 1) != 1) return false;
+  return f16_skinny_tile(M, n, glu, num_cus) != 0;
+}
+
+hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
+                                     bool out_f16, int num_cus, hipStream_t st) {
+  if (!glu) n_out = N, out_f16 = true;
+  switch (f16_skinny_tile(M, n_out, glu != 0, num_cus)) {
+    case 11: return launch_skinny_f16<1, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    case 21: return launch_skinny_f16<2, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    case 12: return launch_skinny_f16<1, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+  }
+  return hipErrorInvalidValue;
+}
