@@ -71,7 +71,7 @@ def test_skinny_f16(rk, orc, m, k, n):
 
 @pytest.mark.parametrize("glu", ["silu", "gelu"])
 @pytest.mark.parametrize("m,k,n", [(1, 64, 3), (16, 1152, 40), (32, 416, 64), (29, 3072, 17),
-                                   (24, 128, 1500), (128, 256, 72), (9, 96, 4600)])
+                                   (24, 128, 1500), (128, 256, 72), (9, 96, 4000)])
 def test_skinny_glu_equals_products_then_glue(rk, orc, m, k, n, glu):
     """The fused forms give what the two plain products and the glue op give, bit for bit."""
     note(f"skinny gate|up m={m} k={k} n={n} {glu}")
