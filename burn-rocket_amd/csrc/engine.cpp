@@ -1199,21 +1199,13 @@ int attn_check(int64_t n_q, int64_t n_kv, int n_head, int n_kv_heads, int head_d
   return RK_OK;
 }
 
-// cs: the call's scope, which provides the key-split workspace; null (the
-// no-allocation entry) launches without a key split.
-int attn_run(const void *q, const void *k, const void *vt, void *out, int64_t n_q, int64_t n_kv,
-             int64_t n_kv_pad, int n_head, int n_kv_heads, int head_dim, float scale, float softcap,
-             int mode, int64_t window, int64_t q0, int64_t k0, bool head_major, hipStream_t st,
-             const char *op, CallScope *cs, int64_t q_ts = 0, int64_t k_ts = 0, int64_t o_ts = 0) {
-  // K and Vᵀ of one kv head are addressed with 32-bit byte offsets.
-  const int64_t k_tok = head_major ? head_dim : (k_ts ? k_ts : (int64_t)n_kv_heads * head_dim);
-  if (((n_kv - 1) * k_tok + head_dim) * 2 >= ((int64_t)1 << 31) ||
-      (int64_t)rk_attn_dv_pad(head_dim) * n_kv_pad * 2 >= ((int64_t)1 << 31))
-    return fail(RK_E_SHAPE, op, "one kv head's K rows or Vᵀ reach 2 GiB");
+// The kernels' arguments. Token strides of 0: packed.
+AttnArgs attn_args(const void *q, const void *k, void *out, int64_t n_q, int64_t n_kv, int n_head, int n_kv_heads,
+                   int head_dim, float scale, float softcap, int mode, int64_t window, int64_t q0, int64_t k0,
+                   bool head_major, int64_t q_ts, int64_t k_ts, int64_t o_ts) {
   AttnArgs a{};
   a.q = q;
   a.k = k;
-  a.vt = vt;
   a.out = out;
   if (head_major) {
     a.q_tok_stride = head_dim;
@@ -1232,7 +1224,6 @@ int attn_run(const void *q, const void *k, const void *vt, void *out, int64_t n_
   }
   a.n_q = (int)n_q;
   a.n_kv = (int)n_kv;
-  a.n_kv_pad = (int)n_kv_pad;
   a.n_head = n_head;
   a.n_kv_heads = n_kv_heads;
   a.head_dim = head_dim;
@@ -1243,32 +1234,66 @@ int attn_run(const void *q, const void *k, const void *vt, void *out, int64_t n_
   a.q0 = q0;
   a.k0 = k0;
   a.num_cus = g_eng->num_cus;
+  return a;
+}
+
+// The workspace of a key split: partial states, and arrival counters that
+// start at zero and that every launch leaves at zero (a new counter buffer is
+// zeroed whole: a later launch with more tiles uses counters past this one's).
+int attn_workspace(CallScope &cs, size_t part_bytes, size_t n_cnt, AttnArgs &a, const char *op) {
+  void *part, *cnt;
+  bool fresh = false;
+  const size_t cnt_bytes = std::max<size_t>(n_cnt * 4, 256);
+  RK_TRY(scratch(cs, "attn_part", part_bytes, &part));
+  RK_TRY(scratch(cs, "attn_cnt", cnt_bytes, &cnt, &fresh));
+  if (fresh) HIP_TRY(hipMemsetAsync(cnt, 0, cnt_bytes, cs.st), op);
+  a.part = (float *)part;
+  a.cnt = (unsigned *)cnt;
+  return RK_OK;
+}
+
+// Few query rows: V is read as it lies, no Vᵀ. *done: whether the call was one.
+int attn_rows_run(CallScope &cs, AttnArgs a, const void *v, int64_t v_ts, bool *done, const char *op) {
+  *done = rk_attn_rows_fits(a, v_ts);
+  if (!*done) return RK_OK;
+  size_t part_bytes, n_cnt;
+  rk_attn_rows_workspace(a, &part_bytes, &n_cnt);
+  if (n_cnt) RK_TRY(attn_workspace(cs, part_bytes, n_cnt, a, op));
+  HIP_TRY(rk_launch_attention_rows(a, v, v_ts, a.head_dim, cs.st), op);
+  return RK_OK;
+}
+
+// cs: the call's scope, which provides the key-split workspace; null (the
+// no-allocation entry) launches without a key split.
+int attn_run(const void *q, const void *k, const void *vt, void *out, int64_t n_q, int64_t n_kv,
+             int64_t n_kv_pad, int n_head, int n_kv_heads, int head_dim, float scale, float softcap,
+             int mode, int64_t window, int64_t q0, int64_t k0, bool head_major, hipStream_t st,
+             const char *op, CallScope *cs, int64_t q_ts = 0, int64_t k_ts = 0, int64_t o_ts = 0) {
+  // K and Vᵀ of one kv head are addressed with 32-bit byte offsets.
+  const int64_t k_tok = head_major ? head_dim : (k_ts ? k_ts : (int64_t)n_kv_heads * head_dim);
+  if (((n_kv - 1) * k_tok + head_dim) * 2 >= ((int64_t)1 << 31) ||
+      (int64_t)rk_attn_dv_pad(head_dim) * n_kv_pad * 2 >= ((int64_t)1 << 31))
+    return fail(RK_E_SHAPE, op, "one kv head's K rows or Vᵀ reach 2 GiB");
+  AttnArgs a = attn_args(q, k, out, n_q, n_kv, n_head, n_kv_heads, head_dim, scale, softcap, mode, window, q0, k0,
+                         head_major, q_ts, k_ts, o_ts);
+  a.vt = vt;
+  a.n_kv_pad = (int)n_kv_pad;
   const long split = cs ? rk_attn_split_tiles(a) : 0;
-  if (split > 0) {
-    // Partial states (two per split tile) and arrival counters. The counters
-    // start at zero and every launch leaves them at zero.
-    // A new counter buffer is zeroed whole: a later launch with more query
-    // tiles uses counters past this one's.
-    void *part, *cnt;
-    bool fresh = false;
-    const size_t cnt_bytes = std::max<size_t>((size_t)split * 4, 256);
-    RK_TRY(scratch(*cs, "attn_part", (size_t)split * 2 * rk_attn_split_floats(head_dim) * 4, &part));
-    RK_TRY(scratch(*cs, "attn_cnt", cnt_bytes, &cnt, &fresh));
-    if (fresh) HIP_TRY(hipMemsetAsync(cnt, 0, cnt_bytes, st), op);
-    a.part = (float *)part;
-    a.cnt = (unsigned *)cnt;
+  if (split > 0) {  // two states per split tile
+    RK_TRY(attn_workspace(*cs, (size_t)split * 2 * rk_attn_split_floats(head_dim) * 4, (size_t)split, a, op));
     a.n_split = (int)split;
   }
   HIP_TRY(rk_launch_attention(a, st), op);
   return RK_OK;
 }
 
-// Token-major attention on device buffers: Vᵀ into scratch, then the kernel.
+// Token-major attention on device buffers: few rows directly (unless few_rows is
+// false), else Vᵀ into scratch, then the kernel.
 int attn_dev_impl(CallScope &cs, const void *q, const void *k, const void *v, int64_t n_q,
                   int64_t n_kv, int n_head, int n_kv_heads, int head_dim, float scale,
                   float softcap, int mode, int64_t window, int64_t q0, int64_t k0, void *out,
                   const char *op, int64_t q_ts = 0, int64_t k_ts = 0, int64_t v_ts = 0,
-                  int64_t o_ts = 0) {
+                  int64_t o_ts = 0, bool few_rows = true) {
   // Head dims of the reference's contract (head_dim % 32, attn/mod.rs:1443)
   // between the kernel widths (160, 192, 224) run zero-padded to 256 on
   // packed token-major operands: zero q/k columns leave the scores, zero V
@@ -1296,7 +1321,7 @@ int attn_dev_impl(CallScope &cs, const void *q, const void *k, const void *v, in
       HIP_TRY(hipMemcpy2DAsync(t.dst, w, t.src, hd, hd, t.rows, hipMemcpyDeviceToDevice, cs.st), op);
     }
     RK_TRY(attn_dev_impl(cs, qp, kp, vp, n_q, n_kv, n_head, n_kv_heads, pad_w, scale, softcap, mode,
-                         window, q0, k0, op_, op));
+                         window, q0, k0, op_, op, 0, 0, 0, 0, few_rows));
     HIP_TRY(hipMemcpy2DAsync(out, hd, op_, w, hd, (size_t)n_q * n_head, hipMemcpyDeviceToDevice, cs.st),
             op);
     return RK_OK;
@@ -1306,6 +1331,14 @@ int attn_dev_impl(CallScope &cs, const void *q, const void *k, const void *v, in
   const int64_t n_kv_pad = round_up_i(n_kv, rk_attn_kv_tile());
   if ((int64_t)dvp * n_kv_pad * 2 >= ((int64_t)1 << 31))
     return fail(RK_E_SHAPE, op, "one kv head's Vᵀ reaches 2 GiB");
+  if (few_rows) {
+    bool done;
+    RK_TRY(attn_rows_run(cs,
+                         attn_args(q, k, out, n_q, n_kv, n_head, n_kv_heads, head_dim, scale, softcap, mode, window, q0,
+                                   k0, false, q_ts, k_ts, o_ts),
+                         v, v_ts ? v_ts : (int64_t)n_kv_heads * head_dim, &done, op));
+    if (done) return RK_OK;
+  }
   void *vt;
   RK_TRY(scratch(cs, "attn_vt", (size_t)n_kv_heads * dvp * n_kv_pad * 2, &vt));
   HIP_TRY(rk_launch_v_transpose(v, v_ts ? v_ts : (int64_t)n_kv_heads * head_dim, head_dim,
@@ -1424,8 +1457,10 @@ extern "C" int rk_attention(const float *q, const float *k, const float *v, int6
     HIP_TRY(rk_launch_f32_to_f16_checked(q32, q16, (int64_t)nq_el, flag, st), op);
     HIP_TRY(rk_launch_f32_to_f16_checked(k32, k16, (int64_t)nk_el, flag, st), op);
     HIP_TRY(rk_launch_f32_to_f16(v32, v16, (int64_t)nk_el, st), op);
+    // (one kernel at every size, the one rk_flash_attn_f16 runs: the host
+    // entries agree bit for bit, and their time is the copies')
     RK_TRY(attn_dev_impl(cs, q16, k16, v16, n_q, n_kv, n_head, n_kv_heads, head_dim, scale, softcap,
-                         mode, window, q0, k0, o16, op));
+                         mode, window, q0, k0, o16, op, 0, 0, 0, 0, false));
     // the output overwrites q's f32 copy, which is no longer read
     HIP_TRY(rk_launch_f16_to_f32(o16, q32, (int64_t)nq_el, st), op);
     return RK_OK;
@@ -2285,12 +2320,23 @@ extern "C" int rk_attention_qkv_dev(void *qkv, int64_t s, int64_t row_stride, in
   CallScope cs(st);
   const int dvp = rk_attn_dv_pad(head_dim);
   const int64_t n_kv_pad = round_up_i(s, rk_attn_kv_tile());
+  const uint16_t *kp = (const uint16_t *)qkv + (int64_t)n_head * head_dim, *vp = kp + (int64_t)n_kv_heads * head_dim;
+  const AttnArgs rows = attn_args(qkv, kp, out, s, s, n_head, n_kv_heads, head_dim, scale, softcap, mode, window, q0, k0,
+                                  false, row_stride, row_stride, out_stride);
+  if (rk_attn_rows_fits(rows, row_stride)) {
+    HIP_TRY(rk_launch_qk_norm_rope(qkv, row_stride, (int)s, n_head, n_kv_heads, head_dim, q_norm_w, k_norm_w,
+                                   (float)eps, cos, sin, cs_dtype, RK_DTYPE_F16, st), name);
+    bool done;
+    RK_TRY(attn_rows_run(cs, rows, vp, row_stride, &done, name));
+    g_eng->calls++;
+    return RK_OK;
+  }
   void *vt;
   RK_TRY(scratch(cs, "attn_vt", (size_t)n_kv_heads * dvp * n_kv_pad * 2, &vt));
   HIP_TRY(rk_launch_qk_norm_rope(qkv, row_stride, (int)s, n_head, n_kv_heads, head_dim, q_norm_w,
                                  k_norm_w, (float)eps, cos, sin, cs_dtype, RK_DTYPE_F16, st, vt,
                                  (int)n_kv_pad, dvp), name);
-  RK_TRY(attn_run(qkv, (const uint16_t *)qkv + (int64_t)n_head * head_dim, vt, out, s, s, n_kv_pad,
+  RK_TRY(attn_run(qkv, kp, vt, out, s, s, n_kv_pad,
                   n_head, n_kv_heads, head_dim, scale, softcap, mode, window, q0, k0, false, st,
                   name, &cs, row_stride, row_stride, out_stride));
   g_eng->calls++;
