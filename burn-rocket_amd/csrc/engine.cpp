@@ -115,6 +115,11 @@ struct Engine {
   double convert_s = 0, device_s = 0;
   uint64_t calls = 0;
   rkstage::HostStage stage;  // page-locked staging of the host-buffer entries
+  // Page-locked lists of rk_moe_experts_dev, grown to the largest call and
+  // given back by rk_clear_scratch. Each call ends with its stream
+  // synchronized, so none is in flight between calls.
+  uint8_t *moe_pin = nullptr;
+  size_t moe_pin_bytes = 0;
   uint64_t epoch = 0;        // rk_trim_scratch: scratch not used since the last trim goes
 };
 
@@ -383,7 +388,7 @@ extern "C" int rk_mem_stats(rk_mem_stats_t *out) {
     if (kv.first.rfind("at", 0) == 0 || kv.first.rfind("fa_", 0) == 0)
       out->attention_bytes += kv.second.bytes;
   }
-  out->host_bytes = g_eng->stage.pinned_bytes();
+  out->host_bytes = g_eng->stage.pinned_bytes() + g_eng->moe_pin_bytes;
   return RK_OK;
 }
 
@@ -416,8 +421,13 @@ extern "C" int rk_trim_scratch_to(uint64_t budget) {
     RK_TRY(free_scratch(o.second, "rk_trim_scratch_to"));
     total -= o.first;
   }
-  // A zero budget also returns the page-locked staging slots.
-  if (budget == 0) HIP_TRY(g_eng->stage.release(), "rk_trim_scratch_to");
+  // A zero budget also returns the page-locked host memory.
+  if (budget == 0) {
+    HIP_TRY(g_eng->stage.release(), "rk_trim_scratch_to");
+    if (g_eng->moe_pin) HIP_TRY(hipHostFree(g_eng->moe_pin), "rk_trim_scratch_to");
+    g_eng->moe_pin = nullptr;
+    g_eng->moe_pin_bytes = 0;
+  }
   return RK_OK;
 }
 
@@ -1816,6 +1826,7 @@ struct MoePlan {
   int32_t *slot = nullptr;    // [s, top_k] bucket rows of a token, ascending expert id
   MoeTile *tiles = nullptr;   // [n_tiles] in expert order (down)
   MoeTile *tiles_gu = nullptr;  // [n_tiles] the same tiles, longest first (gate|up)
+  void *block = nullptr;      // the lists' allocation, when the plan owns it
   uint64_t weight = 0;        // expert stack the plan was made for
   // Streams of the runs that read the lists: a library stream is
   // synchronized when the plan is destroyed; a caller's stream gets an event
@@ -1827,91 +1838,123 @@ void plan_free(MoePlan *p) {
   if (!p) return;
   for (auto &u : p->uses)
     if (u.second) (void)hipEventDestroy(u.second);
-  (void)hipFree(p->tok);
-  (void)hipFree(p->roww);
-  (void)hipFree(p->slot);
-  (void)hipFree(p->tiles);
-  (void)hipFree(p->tiles_gu);
+  (void)hipFree(p->block);
   delete p;
 }
 
-// Bucket the (token, slot) pairs per expert in ascending token order
-// (engine.rs:292-305), list tiles of ≤ rk_moe_tile_rows() rows (two tiles of
-// one expert sit next to each other, so the second read of its weights is
-// mostly served from cache), and sort each token's slot rows by
-// expert id for the combine; the lists are copied into the plan's buffers.
-int moe_plan(const Weight &w, int64_t s, int top_k, const uint32_t *ids, const float *wts,
-             MoePlan *plan, hipStream_t st) {
-  const char *op = "rk_moe_plan";
+// The lists of a call in one block, as byte offsets (tok at 0).
+struct MoeLists {
+  int64_t s = 0;
+  int top_k = 0;
+  int64_t rows = 0;
+  int n_tiles = 0, tile_rows = 128;
+  std::vector<int64_t> off;  // [n_experts + 1] first bucket row of each expert
+  size_t roww = 0, tiles = 0, tiles_gu = 0, slot = 0, bytes = 0;
+};
+
+// Checks the ids and sizes the lists: tiles of ≤ rk_moe_tile_rows() rows (two
+// tiles of one expert sit next to each other, so the second read of its
+// weights is mostly served from cache).
+int moe_lists(const Weight &w, int64_t s, int top_k, const uint32_t *ids, MoeLists *l) {
   const int E = w.n_experts;
-  std::vector<int64_t> count(E, 0);
-  for (int64_t i = 0; i < s * top_k; ++i) {
-    if (ids[i] >= (uint32_t)E) return fail(RK_E_SHAPE, op, "expert id out of range");
-    count[ids[i]]++;
+  l->s = s;
+  l->top_k = top_k;
+  l->rows = s * top_k;
+  l->tile_rows = rk_moe_tile_rows();
+  l->off.assign(E + 1, 0);
+  for (int64_t i = 0; i < l->rows; ++i) {
+    if (ids[i] >= (uint32_t)E) return fail(RK_E_SHAPE, "rk_moe_plan", "expert id out of range");
+    l->off[ids[i] + 1]++;
   }
-  std::vector<int64_t> off(E + 1, 0);
-  for (int e = 0; e < E; ++e) off[e + 1] = off[e] + count[e];
-  const int64_t R = off[E];
-  std::vector<int32_t> tok(R), slot(s * top_k);
-  std::vector<float> roww(R);
-  std::vector<int64_t> fill(off.begin(), off.end() - 1);
-  for (int64_t t = 0; t < s; ++t)
-    for (int j = 0; j < top_k; ++j) {
-      const int e = (int)ids[t * top_k + j];
-      const int64_t row = fill[e]++;
-      tok[row] = (int32_t)t;
-      roww[row] = wts[t * top_k + j];
-      slot[t * top_k + j] = (int32_t)row;
-    }
-  // Rows of one expert are contiguous and expert-major, so ordering a token's
-  // slots by row is ordering them by expert id.
-  for (int64_t t = 0; t < s; ++t) std::sort(slot.begin() + t * top_k, slot.begin() + (t + 1) * top_k);
-  std::vector<MoeTile> tiles;
-  const int tr = rk_moe_tile_rows();
-  for (int e = 0; e < E; ++e)
-    for (int64_t r = off[e]; r < off[e + 1]; r += tr)
-      tiles.push_back(MoeTile{e, (int)r, (int)std::min<int64_t>(tr, off[e + 1] - r)});
-  // gate|up takes the tiles longest first (a tile's time grows with its
-  // 32-row blocks; ties in expert order): the kernels put tile t on XCD t mod 8
-  // and each XCD takes its tiles in list order, so every XCD runs its longest
-  // tiles first and the short ones fill the last round. Per-workgroup
-  // timestamps of a 30B-A3B expert layer (1024 tokens, top-8 of 128) on
-  // MI355X: gate|up 148 -> 141 us; the down kernel in the same order took
-  // 98 -> 107 us (its shortest tiles, run last, then carry most of the
-  // combine's merges), so it keeps expert order. Neither result depends on
-  // the order: the combine sums a token's rows in ascending expert id.
-  std::vector<MoeTile> tiles_gu(tiles);
-  std::stable_sort(tiles_gu.begin(), tiles_gu.end(),
-                   [](const MoeTile &x, const MoeTile &y) { return (x.rows + 31) / 32 > (y.rows + 31) / 32; });
-  HIP_TRY(hipMalloc((void **)&plan->tok, std::max<size_t>(R, 1) * 4), op);
-  HIP_TRY(hipMalloc((void **)&plan->roww, std::max<size_t>(R, 1) * 4), op);
-  HIP_TRY(hipMalloc((void **)&plan->slot, std::max<size_t>(slot.size(), 1) * 4), op);
-  HIP_TRY(hipMalloc((void **)&plan->tiles, std::max<size_t>(tiles.size(), 1) * sizeof(MoeTile)), op);
-  HIP_TRY(hipMalloc((void **)&plan->tiles_gu, std::max<size_t>(tiles.size(), 1) * sizeof(MoeTile)), op);
-  if (R) {
-    HIP_TRY(hipMemcpyAsync(plan->tok, tok.data(), R * 4, hipMemcpyHostToDevice, st), op);
-    HIP_TRY(hipMemcpyAsync(plan->roww, roww.data(), R * 4, hipMemcpyHostToDevice, st), op);
-    HIP_TRY(hipMemcpyAsync(plan->tiles, tiles.data(), tiles.size() * sizeof(MoeTile),
-                           hipMemcpyHostToDevice, st),
-            op);
-    HIP_TRY(hipMemcpyAsync(plan->tiles_gu, tiles_gu.data(), tiles_gu.size() * sizeof(MoeTile),
-                           hipMemcpyHostToDevice, st),
-            op);
+  for (int e = 0; e < E; ++e) {
+    l->n_tiles += (int)((l->off[e + 1] + l->tile_rows - 1) / l->tile_rows);
+    l->off[e + 1] += l->off[e];
   }
-  if (!slot.empty())
-    HIP_TRY(hipMemcpyAsync(plan->slot, slot.data(), slot.size() * 4, hipMemcpyHostToDevice, st), op);
-  // The host vectors die at return: finish the copies first.
-  HIP_TRY(hipStreamSynchronize(st), op);
-  plan->s = s;
-  plan->top_k = top_k;
-  plan->rows = R;
-  plan->n_tiles = (int)tiles.size();
-  plan->tile_rows = tr;
+  const auto pad = [](size_t b) { return (b + 15) / 16 * 16; };
+  l->roww = pad((size_t)l->rows * 4);
+  l->tiles = 2 * l->roww;
+  l->tiles_gu = l->tiles + pad((size_t)l->n_tiles * sizeof(MoeTile));
+  l->slot = l->tiles_gu + pad((size_t)l->n_tiles * sizeof(MoeTile));
+  l->bytes = l->slot + pad((size_t)l->rows * 4);
   return RK_OK;
 }
 
+// The lists up to `slot`: the (token, slot) pairs bucketed per expert in
+// ascending token order (engine.rs:292-305), and the tiles.
+// gate|up takes the tiles longest first (a tile's time grows with its
+// 32-row blocks; ties in expert order): the kernels put tile t on XCD t mod 8
+// and each XCD takes its tiles in list order, so every XCD runs its longest
+// tiles first and the short ones fill the last round. Per-workgroup
+// timestamps of a 30B-A3B expert layer (1024 tokens, top-8 of 128) on
+// MI355X: gate|up 148 -> 141 us; the down kernel in the same order took
+// 98 -> 107 us (its shortest tiles, run last, then carry most of the
+// combine's merges), so it keeps expert order. Neither result depends on
+// the order: the combine sums a token's rows in ascending expert id.
+void moe_fill_rows(const MoeLists &l, const uint32_t *ids, const float *wts, uint8_t *host) {
+  int32_t *tok = (int32_t *)host;
+  float *roww = (float *)(host + l.roww);
+  std::vector<int64_t> fill(l.off.begin(), l.off.end() - 1);
+  for (int64_t t = 0, i = 0; t < l.s; ++t)
+    for (int j = 0; j < l.top_k; ++j, ++i) {
+      const int64_t row = fill[ids[i]]++;
+      tok[row] = (int32_t)t;
+      roww[row] = wts[i];
+    }
+  MoeTile *tiles = (MoeTile *)(host + l.tiles), *gu = (MoeTile *)(host + l.tiles_gu);
+  int n = 0;
+  for (int e = 0; e + 1 < (int)l.off.size(); ++e)
+    for (int64_t r = l.off[e]; r < l.off[e + 1]; r += l.tile_rows)
+      tiles[n++] = MoeTile{e, (int)r, (int)std::min<int64_t>(l.tile_rows, l.off[e + 1] - r)};
+  for (int blocks = l.tile_rows / 32, m = 0; blocks >= 1; --blocks)
+    for (int i = 0; i < n; ++i)
+      if ((tiles[i].rows + 31) / 32 == blocks) gu[m++] = tiles[i];
+}
+
+// Each token's bucket rows for the combine. Rows of one expert are contiguous
+// and expert-major, so taking the rows in order lists a token's by expert id.
+void moe_fill_slots(const MoeLists &l, uint8_t *host) {
+  const int32_t *tok = (const int32_t *)host;
+  int32_t *slot = (int32_t *)(host + l.slot);
+  std::vector<int32_t> n(l.s, 0);
+  for (int64_t row = 0; row < l.rows; ++row) slot[(int64_t)tok[row] * l.top_k + n[tok[row]]++] = (int32_t)row;
+}
+
+// Points the plan at a device block that holds (or will hold) the lists.
+void moe_bind(const MoeLists &l, uint8_t *dev, MoePlan *plan) {
+  plan->s = l.s;
+  plan->top_k = l.top_k;
+  plan->rows = l.rows;
+  plan->n_tiles = l.n_tiles;
+  plan->tile_rows = l.tile_rows;
+  plan->tok = (int32_t *)dev;
+  plan->roww = (float *)(dev + l.roww);
+  plan->tiles = (MoeTile *)(dev + l.tiles);
+  plan->tiles_gu = (MoeTile *)(dev + l.tiles_gu);
+  plan->slot = (int32_t *)(dev + l.slot);
+}
+
+// A plan with lists of its own on the device.
+int moe_plan(const Weight &w, int64_t s, int top_k, const uint32_t *ids, const float *wts,
+             MoePlan *plan, hipStream_t st) {
+  const char *op = "rk_moe_plan";
+  MoeLists l;
+  RK_TRY(moe_lists(w, s, top_k, ids, &l));
+  HIP_TRY(hipMalloc(&plan->block, l.bytes), op);
+  std::vector<uint8_t> host(l.bytes);
+  moe_fill_rows(l, ids, wts, host.data());
+  moe_fill_slots(l, host.data());
+  HIP_TRY(hipMemcpyAsync(plan->block, host.data(), l.bytes, hipMemcpyHostToDevice, st), op);
+  // The host vector dies at return: finish the copy first.
+  HIP_TRY(hipStreamSynchronize(st), op);
+  moe_bind(l, (uint8_t *)plan->block, plan);
+  return RK_OK;
+}
+
+// lists (when given) enqueues the plan's lists: called with 0 before the launch
+// that reads all but `slot`, with 1 before the one that reads `slot`.
 int moe_run(CallScope &cs, const Weight &w, const MoePlan &plan, const float *x, float *y,
-            float *act_out = nullptr, bool accumulate = false) {
+            float *act_out = nullptr, bool accumulate = false,
+            const std::function<int(int)> &lists = nullptr) {
   hipStream_t st = cs.st;
   const int64_t H = w.hidden, I = w.inter, S = plan.s, R = std::max<int64_t>(plan.rows, 1);
   const int64_t KBh = H / 32, KBi = I / 32;  // 32-value activation groups per row
@@ -1935,6 +1978,7 @@ int moe_run(CallScope &cs, const Weight &w, const MoePlan &plan, const float *x,
   // x and the silu·up rows are quantized per row per 32-value group, as the
   // reference's expert workers do (engine.rs:1005-1006, 1034-1035).
   HIP_TRY(rk_launch_quantize_rows(x, S, H, 32, (int8_t *)xq, (float *)xs, st), op);
+  if (lists) RK_TRY(lists(0));
   HIP_TRY(rk_launch_moe_gemm_gu(plan.tile_rows, (const int8_t *)xq, (const float *)xs, (int)KBh, plan.tok, S,
                                 plan.tiles_gu, plan.n_tiles, w.gu_codes, w.gu_scales,
                                 moe_gu_code_stride(w), 2 * I * w.gu_ws_stride, w.gu_ws_stride,
@@ -1943,6 +1987,7 @@ int moe_run(CallScope &cs, const Weight &w, const MoePlan &plan, const float *x,
   if (!y) return RK_OK;  // stage 1 only
   HIP_TRY(rk_launch_quantize_rows((const float *)act, plan.rows, I, 32, (int8_t *)aq, (float *)as, st),
           op);
+  if (lists) RK_TRY(lists(1));
   MoeCombine cmb;
   cmb.tok = plan.tok;
   cmb.slot = plan.slot;
@@ -1997,12 +2042,40 @@ int moe_experts(rk_weight_id id, const float *x, int64_t s, int top_k, const uin
   if (!x || !y || !ids || !wts) return fail(RK_E_SHAPE, op, "null buffer");
   hipStream_t st = pick(stream);
   CallScope cs(st);
-  MoePlan *plan = new MoePlan();
-  int rc = moe_plan(*w, s, top_k, ids, wts, plan, st);
-  if (rc == RK_OK) rc = moe_run(cs, *w, *plan, x, y, nullptr, accumulate);
-  // The plan's lists must outlive the kernels that read them.
-  hipError_t e = hipStreamSynchronize(st);
-  plan_free(plan);
+  // The lists go from page-locked memory to scratch, long ones in two copies, so
+  // that the host fills them while the GPU works: the rows during the quantizer
+  // of x, the slots during gate|up. (With allocations, pageable copies and frees of
+  // five lists per call, 8 tokens on 128 experts took 122 us for 78 us of
+  // kernels and 1024 tokens 336 us for 256 us on MI355X; now 100 and 304.)
+  MoeLists l;
+  RK_TRY(moe_lists(*w, s, top_k, ids, &l));
+  if (g_eng->moe_pin_bytes < l.bytes) {
+    if (g_eng->moe_pin) HIP_TRY(hipHostFree(g_eng->moe_pin), op);
+    g_eng->moe_pin = nullptr;
+    g_eng->moe_pin_bytes = 0;
+    const size_t want = (l.bytes + 65535) / 65536 * 65536;
+    HIP_TRY(hipHostMalloc((void **)&g_eng->moe_pin, want, hipHostMallocDefault), op);
+    g_eng->moe_pin_bytes = want;
+  }
+  uint8_t *host = g_eng->moe_pin, *dev;
+  RK_TRY(scratch(cs, "moe_lists", l.bytes, (void **)&dev));
+  MoePlan plan;
+  moe_bind(l, dev, &plan);
+  const int rc = moe_run(cs, *w, plan, x, y, nullptr, accumulate, [&](int part) {
+    const bool one = l.rows <= 2048;  // a second copy costs more than filling the slots first
+    if (part == 0) {
+      moe_fill_rows(l, ids, wts, host);
+      if (one) moe_fill_slots(l, host);
+      HIP_TRY(hipMemcpyAsync(dev, host, one ? l.bytes : l.slot, hipMemcpyHostToDevice, st), op);
+    } else if (!one) {
+      moe_fill_slots(l, host);
+      HIP_TRY(hipMemcpyAsync(dev + l.slot, host + l.slot, l.bytes - l.slot, hipMemcpyHostToDevice, st), op);
+    }
+    return (int)RK_OK;
+  });
+  // The page-locked lists must outlive the copies (also of a call that failed
+  // half way).
+  const hipError_t e = hipStreamSynchronize(st);
   if (rc != RK_OK) return rc;
   HIP_TRY(e, op);
   g_eng->calls++;

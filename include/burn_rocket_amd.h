@@ -115,7 +115,7 @@ int rk_stats_reset(void);
  * the largest call that used it; attention_bytes is the part the attention
  * entries use (the reference's attention_bo_bytes, the rest its
  * matmul_bo_bytes); host_bytes is the page-locked staging of the host-buffer
- * entries (its *_host_bytes). */
+ * entries (its *_host_bytes) and the bucket lists of rk_moe_experts_dev. */
 typedef struct {
   uint64_t weights_bytes;   /* resident weights */
   uint64_t scratch_bytes;   /* device scratch, all buffers */
