@@ -1821,6 +1821,7 @@ struct MoePlan {
   int64_t rows = 0;
   int n_tiles = 0;
   int tile_rows = 128;        // rows per tile at most (the kernels' tile size)
+  int max_rows = 128;         // rows of the longest tile
   int32_t *tok = nullptr;     // [rows] token of each bucket row
   float *roww = nullptr;      // [rows] router weight of each bucket row
   int32_t *slot = nullptr;    // [s, top_k] bucket rows of a token, ascending expert id
@@ -1847,7 +1848,7 @@ struct MoeLists {
   int64_t s = 0;
   int top_k = 0;
   int64_t rows = 0;
-  int n_tiles = 0, tile_rows = 128;
+  int n_tiles = 0, tile_rows = 128, max_rows = 0;
   std::vector<int64_t> off;  // [n_experts + 1] first bucket row of each expert
   size_t roww = 0, tiles = 0, tiles_gu = 0, slot = 0, bytes = 0;
 };
@@ -1868,6 +1869,7 @@ int moe_lists(const Weight &w, int64_t s, int top_k, const uint32_t *ids, MoeLis
   }
   for (int e = 0; e < E; ++e) {
     l->n_tiles += (int)((l->off[e + 1] + l->tile_rows - 1) / l->tile_rows);
+    l->max_rows = (int)std::max<int64_t>(l->max_rows, std::min<int64_t>(l->off[e + 1], l->tile_rows));
     l->off[e + 1] += l->off[e];
   }
   const auto pad = [](size_t b) { return (b + 15) / 16 * 16; };
@@ -1926,6 +1928,7 @@ void moe_bind(const MoeLists &l, uint8_t *dev, MoePlan *plan) {
   plan->rows = l.rows;
   plan->n_tiles = l.n_tiles;
   plan->tile_rows = l.tile_rows;
+  plan->max_rows = l.max_rows;
   plan->tok = (int32_t *)dev;
   plan->roww = (float *)(dev + l.roww);
   plan->tiles = (MoeTile *)(dev + l.tiles);
@@ -1979,7 +1982,7 @@ int moe_run(CallScope &cs, const Weight &w, const MoePlan &plan, const float *x,
   // reference's expert workers do (engine.rs:1005-1006, 1034-1035).
   HIP_TRY(rk_launch_quantize_rows(x, S, H, 32, (int8_t *)xq, (float *)xs, st), op);
   if (lists) RK_TRY(lists(0));
-  HIP_TRY(rk_launch_moe_gemm_gu(plan.tile_rows, (const int8_t *)xq, (const float *)xs, (int)KBh, plan.tok, S,
+  HIP_TRY(rk_launch_moe_gemm_gu(plan.tile_rows, plan.max_rows, (const int8_t *)xq, (const float *)xs, (int)KBh, plan.tok, S,
                                 plan.tiles_gu, plan.n_tiles, w.gu_codes, w.gu_scales,
                                 moe_gu_code_stride(w), 2 * I * w.gu_ws_stride, w.gu_ws_stride,
                                 (int)(2 * I), (int)H, (float *)act, st),
@@ -1996,7 +1999,7 @@ int moe_run(CallScope &cs, const Weight &w, const MoePlan &plan, const float *x,
   cmb.n_tok = (int)S;
   cmb.top_k = plan.top_k;
   cmb.accumulate = accumulate ? 1 : 0;
-  HIP_TRY(rk_launch_moe_gemm_down(plan.tile_rows, (const int8_t *)aq, (const float *)as, (int)KBi, plan.rows,
+  HIP_TRY(rk_launch_moe_gemm_down(plan.tile_rows, plan.max_rows, (const int8_t *)aq, (const float *)as, (int)KBi, plan.rows,
                                   plan.tiles, plan.n_tiles, w.dn_codes, w.dn_scales,
                                   moe_dn_code_stride(w), H * w.dn_ws_stride, w.dn_ws_stride, (int)H,
                                   (int)I, plan.roww, (float *)yb, cmb, st),

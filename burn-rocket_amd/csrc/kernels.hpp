@@ -214,8 +214,9 @@ struct MoeTile {
 // scales are per row per 32-value group: [a_rows, stride] with stride = K/32.
 // Tiles hold at most tile_rows (64 or 128) bucket rows: rk_moe_tile_rows() is
 // the size a new plan lists (RK_MOE_ROWS), the launches take the plan's.
+// max_rows: the rows of the longest tile.
 int rk_moe_tile_rows();
-hipError_t rk_launch_moe_gemm_gu(int tile_rows, const int8_t *xq, const float *xs, int xs_stride,
+hipError_t rk_launch_moe_gemm_gu(int tile_rows, int max_rows, const int8_t *xq, const float *xs, int xs_stride,
                                  const int32_t *tok, int64_t s, const MoeTile *tiles, int n_tiles, const int8_t *w,
                                  const float *ws, int64_t w_stride_e, int64_t ws_stride_e,
                                  int ws_stride, int N, int K, float *act, hipStream_t st);
@@ -234,7 +235,7 @@ struct MoeCombine {
   int accumulate = 0;             // 1: y += the sum (onto the residual); 0: y = the sum
   int n_tiles = 0;                // set by the launcher
 };
-hipError_t rk_launch_moe_gemm_down(int tile_rows, const int8_t *aq, const float *as, int as_stride, int64_t rows,
+hipError_t rk_launch_moe_gemm_down(int tile_rows, int max_rows, const int8_t *aq, const float *as, int as_stride, int64_t rows,
                                    const MoeTile *tiles, int n_tiles, const int8_t *w, const float *ws,
                                    int64_t w_stride_e, int64_t ws_stride_e, int ws_stride,
                                    int N, int K, const float *row_w, float *yb, const MoeCombine &cmb,

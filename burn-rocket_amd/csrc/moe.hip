@@ -88,6 +88,160 @@ __device__ __forceinline__ void bdma4(rsrc_t r, void *lds_base, uint32_t voff, u
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, LDS_PTR(lds_base), 4, voff, soff, 0, 0);
 }
 
+// The results of a tile: act = silu(g)·u (gate|up), or the rows times their
+// router weight and the combine (down). facc holds NR of the 16 registers of
+// each 32-row block (rows 8·(r/4) + 4·(lane/32) + r%4), the wave's 32 columns
+// from n0. s_rw: the rows' router weights; s_free: room for BM·9 + 1 ints.
+template <bool GU, int NW, int NRB, int NR>
+__device__ __forceinline__ void moe_epilogue(const floatx16 (&facc)[NRB], const MoeTile &tile, int64_t a_rows, int N,
+                                             int n0, const float *s_rw, void *s_free, float *__restrict__ out,
+                                             int out_ld, const MoeCombine &cmb) {
+  constexpr int BM = 32 * NRB;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fcol = lane & 31, fh = lane >> 5;
+  // Epilogue: lane holds rows 8·(r/4) + 4·(lane/32) + r%4 of each 32-row
+  // block, column lane%32 of the wave's 32 columns.
+  const int col = n0 + wave * 32 + fcol;
+  constexpr int SC1 = 16;  // cache policy bit: device scope
+  const rsrc_t ryb = make_rsrc(out + (int64_t)tile.row0 * out_ld, (int64_t)tile.rows * out_ld * 4);
+#pragma unroll
+  for (int i = 0; i < NRB; ++i) {
+    if constexpr (GU) {
+      // Gate column j is in lane j, up column j in lane j + 16 (of each half
+      // wave). For the row pair (r, r+1) the lower lanes finish row r and the
+      // upper lanes row r+1: one swap across the 16-lane halves gives each
+      // lane the gate and up values of its row, so every lane computes one
+      // output.
+      const bool lo = (fcol & 16) == 0;
+#pragma unroll
+      for (int r = 0; r < NR; r += 2) {
+        const int rr = lo ? r : r + 1;
+        const int row = i * 32 + (rr >> 2) * 8 + fh * 4 + (rr & 3);
+        const float v0 = facc[i][r], v1 = facc[i][r + 1];
+        // lower lanes send the gate of row r+1, upper lanes the up of row r
+        const float x = __int_as_float(
+            __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __float_as_int(lo ? v1 : v0)));
+        const float g = lo ? v0 : x, u = lo ? x : v1;
+        if (row < tile.rows && col < N) {
+          const int c = (n0 + wave * 32) / 2 + (fcol & 15);
+          out[(int64_t)(tile.row0 + row) * out_ld + c] = g / (1.0f + exp_rn(-g)) * u;
+        }
+      }
+    } else {
+      // yb rows with device-coherent (sc1) stores: the workgroup that
+      // completes a token may run on another XCD, whose L2 does not see this
+      // one's.
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const int row = i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
+        if (row < tile.rows && col < N)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(facc[i][r] * s_rw[row]), ryb,
+                                                (uint32_t)((row * out_ld + col) * 4), 0, SC1);
+      }
+    }
+  }
+  if constexpr (!GU) {
+    // Combine (engine.rs:317-338). Once every wave's rows are stored, each
+    // row of the tile counts itself in on its token's counter for this
+    // column slice; the row whose count completes the token's top_k rows
+    // belongs to the workgroup that sums them. It resets the counter, so
+    // every launch leaves the counters at zero.
+    WAIT_VMCNT(0);
+    int *s_tok = (int *)s_free;  // [BM] tokens this workgroup completes
+    int *s_sl = s_tok + BM;      // [BM][8] their slot rows (top_k <= 8)
+    int *s_n = s_sl + BM * 8;
+    if (threadIdx.x == 0) *s_n = 0;
+    __syncthreads();
+    const int n_cs = (N + 32 * NW - 1) / (32 * NW), cs = n0 / (32 * NW);
+    const int top_k = cmb.top_k;
+    const bool staged = top_k <= 8;
+    for (int row = threadIdx.x; row < tile.rows; row += NW * 64) {
+      const int t = cmb.tok[tile.row0 + row];
+      unsigned *c = cmb.cnt + (int64_t)t * n_cs + cs;
+      if (atomicAdd(c, 1u) == (unsigned)top_k - 1) {
+        atomicExch(c, 0u);
+        const int idx = atomicAdd(s_n, 1);
+        s_tok[idx] = t;
+        if (staged)
+          for (int j = 0; j < top_k; ++j) s_sl[idx * 8 + j] = cmb.slot[(int64_t)t * top_k + j];
+      }
+    }
+    __syncthreads();
+    // y[t] (+)= Σ_j yb[slot j of t] over the token's rows in ascending
+    // expert id: 4 columns per thread, 8·NW threads per row, U rows per
+    // thread at a time with every row load issued before the first add (the
+    // completing workgroups are the last ones to run, so their loads are
+    // the launch's tail).
+    constexpr int TPR = 8 * NW, NT = NW * 64, RPI = NT / TPR, U = 4;
+    const int n_last = *s_n;
+    const int c = n0 + 4 * ((int)threadIdx.x % TPR);
+    const int sub = (int)threadIdx.x / TPR;
+    const rsrc_t rall = make_rsrc(out, a_rows * out_ld * 4);
+    if (c < N) {
+      if (staged) {
+        // Loads past the token's top_k or past the last row read zeros
+        // (offsets outside the buffer) rather than sitting under a branch,
+        // which would serialise them.
+        const rsrc_t ry = make_rsrc(cmb.y, (int64_t)cmb.n_tok * N * 4);
+        for (int i0 = 0; i0 < n_last; i0 += U * RPI) {
+          floatx4 v[U][8], y0[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int idx = i0 + u * RPI + sub;
+            const bool ok = idx < n_last;
+            const int ic = ok ? idx : 0;
+            const intx4 sa = *(const intx4 *)(s_sl + ic * 8), sb = *(const intx4 *)(s_sl + ic * 8 + 4);
+            const int tk = s_tok[ic];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const int sv = j < 4 ? sa[j & 3] : sb[j & 3];
+              const uint32_t off = (ok && j < top_k) ? (uint32_t)((sv * out_ld + c) * 4) : OOB_OFFSET;
+              v[u][j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rall, off, 0, SC1));
+            }
+            const uint32_t yoff = (ok && cmb.accumulate) ? (uint32_t)((tk * N + c) * 4) : OOB_OFFSET;
+            y0[u] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ry, yoff, 0, 0));
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            floatx4 acc = y0[u];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (j < top_k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = acc[e] + v[u][j][e];
+            const int idx = i0 + u * RPI + sub;
+            if (idx < n_last) *(floatx4 *)(cmb.y + (int64_t)s_tok[idx] * N + c) = acc;
+          }
+        }
+      } else {
+        for (int idx = sub; idx < n_last; idx += RPI) {
+          const int t = s_tok[idx];
+          const int32_t *sl = cmb.slot + (int64_t)t * top_k;
+          float *yr = cmb.y + (int64_t)t * N + c;
+          floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+          if (cmb.accumulate) acc = *(const floatx4 *)yr;
+          for (int j0 = 0; j0 < top_k; j0 += 8) {
+            const int nj = min(8, top_k - j0);
+            floatx4 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (j < nj)
+                v[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       rall, (uint32_t)((sl[j0 + j] * out_ld + c) * 4), 0, SC1));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (j < nj)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = acc[e] + v[j][e];
+          }
+          *(floatx4 *)yr = acc;
+        }
+      }
+    }
+  }
+}
+
 template <bool GU, int NW, int PD, int BM, int NRB>
 __device__ __forceinline__ void moe_body(
     const int8_t *__restrict__ A, const float *__restrict__ AS, int as_stride,
@@ -339,146 +493,7 @@ __device__ __forceinline__ void moe_body(
     fold(ic<0>{}, ic<NRB - 1>{}, dpend, cpend, asp);
   WAIT_VMCNT(0);  // no copy may still be writing LDS when the workgroup ends
 
-  // Epilogue: lane holds rows 8·(r/4) + 4·(lane/32) + r%4 of each 32-row
-  // block, column lane%32 of the wave's 32 columns.
-  const int col = n0 + wave * 32 + fcol;
-  constexpr int SC1 = 16;  // cache policy bit: device scope
-  const rsrc_t ryb = make_rsrc(out + (int64_t)tile.row0 * out_ld, (int64_t)tile.rows * out_ld * 4);
-#pragma unroll
-  for (int i = 0; i < NRB; ++i) {
-    if constexpr (GU) {
-      // Gate column j is in lane j, up column j in lane j + 16 (of each half
-      // wave). For the row pair (r, r+1) the lower lanes finish row r and the
-      // upper lanes row r+1: one swap across the 16-lane halves gives each
-      // lane the gate and up values of its row, so every lane computes one
-      // output.
-      const bool lo = (fcol & 16) == 0;
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        const int rr = lo ? r : r + 1;
-        const int row = i * 32 + (rr >> 2) * 8 + fh * 4 + (rr & 3);
-        const float v0 = facc[i][r], v1 = facc[i][r + 1];
-        // lower lanes send the gate of row r+1, upper lanes the up of row r
-        const float x = __int_as_float(
-            __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __float_as_int(lo ? v1 : v0)));
-        const float g = lo ? v0 : x, u = lo ? x : v1;
-        if (row < tile.rows && col < N) {
-          const int c = (n0 + wave * 32) / 2 + (fcol & 15);
-          out[(int64_t)(tile.row0 + row) * out_ld + c] = g / (1.0f + exp_rn(-g)) * u;
-        }
-      }
-    } else {
-      // yb rows with device-coherent (sc1) stores: the workgroup that
-      // completes a token may run on another XCD, whose L2 does not see this
-      // one's.
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
-        if (row < tile.rows && col < N)
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(facc[i][r] * s_rw[row]), ryb,
-                                                (uint32_t)((row * out_ld + col) * 4), 0, SC1);
-      }
-    }
-  }
-  if constexpr (!GU) {
-    // Combine (engine.rs:317-338). Once every wave's rows are stored, each
-    // row of the tile counts itself in on its token's counter for this
-    // column slice; the row whose count completes the token's top_k rows
-    // belongs to the workgroup that sums them. It resets the counter, so
-    // every launch leaves the counters at zero.
-    WAIT_VMCNT(0);
-    int *s_tok = (int *)(smem + NSLOT * MOE_SLOT + BM * 4);  // [BM] tokens this workgroup completes
-    int *s_sl = s_tok + BM;                                  // [BM][8] their slot rows (top_k <= 8)
-    int *s_n = s_sl + BM * 8;
-    if (threadIdx.x == 0) *s_n = 0;
-    __syncthreads();
-    const int n_cs = (N + 32 * NW - 1) / (32 * NW), cs = n0 / (32 * NW);
-    const int top_k = cmb.top_k;
-    const bool staged = top_k <= 8;
-    for (int row = threadIdx.x; row < tile.rows; row += NW * 64) {
-      const int t = cmb.tok[tile.row0 + row];
-      unsigned *c = cmb.cnt + (int64_t)t * n_cs + cs;
-      if (atomicAdd(c, 1u) == (unsigned)top_k - 1) {
-        atomicExch(c, 0u);
-        const int idx = atomicAdd(s_n, 1);
-        s_tok[idx] = t;
-        if (staged)
-          for (int j = 0; j < top_k; ++j) s_sl[idx * 8 + j] = cmb.slot[(int64_t)t * top_k + j];
-      }
-    }
-    __syncthreads();
-    // y[t] (+)= Σ_j yb[slot j of t] over the token's rows in ascending
-    // expert id: 4 columns per thread, 8·NW threads per row, U rows per
-    // thread at a time with every row load issued before the first add (the
-    // completing workgroups are the last ones to run, so their loads are
-    // the launch's tail).
-    constexpr int TPR = 8 * NW, NT = NW * 64, RPI = NT / TPR, U = 4;
-    const int n_last = *s_n;
-    const int c = n0 + 4 * ((int)threadIdx.x % TPR);
-    const int sub = (int)threadIdx.x / TPR;
-    const rsrc_t rall = make_rsrc(out, a_rows * out_ld * 4);
-    if (c < N) {
-      if (staged) {
-        // Loads past the token's top_k or past the last row read zeros
-        // (offsets outside the buffer) rather than sitting under a branch,
-        // which would serialise them.
-        const rsrc_t ry = make_rsrc(cmb.y, (int64_t)cmb.n_tok * N * 4);
-        for (int i0 = 0; i0 < n_last; i0 += U * RPI) {
-          floatx4 v[U][8], y0[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int idx = i0 + u * RPI + sub;
-            const bool ok = idx < n_last;
-            const int ic = ok ? idx : 0;
-            const intx4 sa = *(const intx4 *)(s_sl + ic * 8), sb = *(const intx4 *)(s_sl + ic * 8 + 4);
-            const int tk = s_tok[ic];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              const int sv = j < 4 ? sa[j & 3] : sb[j & 3];
-              const uint32_t off = (ok && j < top_k) ? (uint32_t)((sv * out_ld + c) * 4) : OOB_OFFSET;
-              v[u][j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rall, off, 0, SC1));
-            }
-            const uint32_t yoff = (ok && cmb.accumulate) ? (uint32_t)((tk * N + c) * 4) : OOB_OFFSET;
-            y0[u] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ry, yoff, 0, 0));
-          }
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            floatx4 acc = y0[u];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (j < top_k)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = acc[e] + v[u][j][e];
-            const int idx = i0 + u * RPI + sub;
-            if (idx < n_last) *(floatx4 *)(cmb.y + (int64_t)s_tok[idx] * N + c) = acc;
-          }
-        }
-      } else {
-        for (int idx = sub; idx < n_last; idx += RPI) {
-          const int t = s_tok[idx];
-          const int32_t *sl = cmb.slot + (int64_t)t * top_k;
-          float *yr = cmb.y + (int64_t)t * N + c;
-          floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-          if (cmb.accumulate) acc = *(const floatx4 *)yr;
-          for (int j0 = 0; j0 < top_k; j0 += 8) {
-            const int nj = min(8, top_k - j0);
-            floatx4 v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (j < nj)
-                v[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                       rall, (uint32_t)((sl[j0 + j] * out_ld + c) * 4), 0, SC1));
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (j < nj)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = acc[e] + v[j][e];
-          }
-          *(floatx4 *)yr = acc;
-        }
-      }
-    }
-  }
+  moe_epilogue<GU, NW, NRB, 16>(facc, tile, a_rows, N, n0, s_rw, s_rw + BM, out, out_ld, cmb);
 }
 
 template <bool GU, int NW, int PD, int BM>
@@ -513,6 +528,115 @@ __global__ __launch_bounds__(NW * 64, 2) void moe_q8_kernel(
       moe_body<GU, NW, PD, BM, NRB>(A, AS, as_stride, tok, a_rows, tile, We, WSe, ws_stride, N, K, n0,
                                     row_w, out, out_ld, cmb, smem);
   });
+}
+
+// Tiles of at most 32 rows (decode steps): no wave shares enough with its
+// neighbours for the LDS ring above to pay. Each wave loads its own MFMA
+// operands, weights and token rows, straight into registers, one stage ahead,
+// and walks K on its own with no barrier: the sums run in the same order with
+// the same roundings (P is exact as a float either way), so the results are
+// those of moe_q8_kernel bit for bit. A few rows fill a few of the 16 result
+// registers: NQ·8 rows fold NQ·4 of them. Few registers and little LDS keep
+// three workgroups on a CU, where the 128-row kernel's two left a second, nearly
+// empty round (30B-A3B experts, 8 tokens: 612 workgroups). HBM-bound on the
+// experts' weights. The planned call on that layer, MI355X, ring kernels -> here:
+// 1 token 38.4 -> 28.9 us, 8 tokens 78.2 -> 62.7 (4.4 TB/s), 64 tokens 152.9 ->
+// 137.5, 128 tokens 156.7 -> 145.0 (4.7 TB/s).
+template <bool GU, int NQ>
+__global__ __launch_bounds__(256, 3) void moe_few_kernel(
+    const int8_t *__restrict__ A, const float *__restrict__ AS, int as_stride,
+    const int32_t *__restrict__ tok, int64_t a_rows, const MoeTile *__restrict__ tiles, int n_col_tiles,
+    const int8_t *__restrict__ W, const float *__restrict__ WS, int64_t w_stride_e,
+    int64_t ws_stride_e, int ws_stride, int N, int K, const float *__restrict__ row_w,
+    float *__restrict__ out, int out_ld, MoeCombine cmb) {
+  constexpr int NW = 4;
+  __shared__ __attribute__((aligned(16))) float s_as[NW][4][32];  // a stage's scales, [block][row]
+  __shared__ float s_rw[32];
+  __shared__ __attribute__((aligned(16))) int s_free[32 * 9 + 4];
+  const int jb = blockIdx.x / 8;  // tile order: see moe_q8_kernel
+  const int t = blockIdx.x % 8 + 8 * (jb / n_col_tiles);
+  if (t >= cmb.n_tiles) return;
+  const MoeTile tile = tiles[t];
+  const int n0 = (jb % n_col_tiles) * 32 * NW;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fcol = lane & 31, fh = lane >> 5;
+  const int KT = (K + 127) / 128, KB = K / 32;
+  if constexpr (!GU) {
+    if (threadIdx.x < 32) s_rw[threadIdx.x] = (int)threadIdx.x < tile.rows ? row_w[tile.row0 + threadIdx.x] : 0.f;
+    __syncthreads();
+  }
+
+  const int KS = ws_stride / 4, cb0 = n0 / 32, ncb = (N + 31) / 32;
+  const rsrc_t ra = make_rsrc(A, a_rows * K);
+  const rsrc_t ras = make_rsrc(AS, a_rows * as_stride * 4);
+  const rsrc_t rw = make_rsrc(W + (int64_t)tile.expert * w_stride_e + (size_t)cb0 * KS * 4096,
+                              (int64_t)(ncb - cb0) * KS * 4096);
+  const rsrc_t rs = make_rsrc(WS + (int64_t)tile.expert * ws_stride_e + (size_t)cb0 * KS * 128,
+                              (int64_t)(ncb - cb0) * KS * 512);
+  const bool row_ok = fcol < tile.rows;
+  const int64_t src = !row_ok ? 0 : GU ? (int64_t)tok[tile.row0 + fcol] : (int64_t)(tile.row0 + fcol);
+  const uint32_t v_a = row_ok ? (uint32_t)(src * K + fh * 16) : OOB_OFFSET;
+  const uint32_t v_as = row_ok && fh == 0 ? (uint32_t)(src * as_stride * 4) : OOB_OFFSET;
+  const uint32_t v_w = (uint32_t)(wave * KS * 4096 + lane * 16), v_ws = (uint32_t)(wave * KS * 512 + fcol * 16);
+
+  struct Stage {
+    intx4 w[4], a[4];
+    floatx4 ws, as;
+  } st[2];
+  auto load = [&](Stage &x, int kt) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) x.w[b] = __builtin_amdgcn_raw_buffer_load_b128(rw, v_w + 1024 * b, kt * 4096, 0);
+    x.ws = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, v_ws, kt * 512, 0));
+#pragma unroll
+    for (int b = 0; b < 4; ++b) x.a[b] = __builtin_amdgcn_raw_buffer_load_b128(ra, v_a + 32 * b, kt * 128, 0);
+    x.as = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ras, v_as, kt * 16, 0));
+  };
+  floatx16 facc[1];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) facc[0][r] = 0.f;
+  auto stage = [&](const Stage &x, int kt) {
+#pragma clang fp contract(off)
+    // (a wave's LDS accesses run in order: nothing waits between these)
+    asm volatile("" ::: "memory");
+    if (fh == 0) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) s_as[wave][b][fcol] = x.as[b];
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      if (kt * 4 + b >= KB) break;  // wave-uniform: K ends inside the stage
+      const intx16 p = __builtin_amdgcn_mfma_i32_32x32x32_i8(x.a[b], x.w[b], intx16{}, 0, 0, 0);
+      const float d = x.ws[b];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const floatx4 as4 = *(const floatx4 *)&s_as[wave][b][q * 8 + fh * 4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * q + e;
+          if constexpr (GU) {  // acc + fl(fl(a_s·w_s)·P), see moe_body
+            const float sc = as4[e] * d;
+            const float y = sc * (float)p[r];
+            facc[0][r] = facc[0][r] + y;
+          } else {
+            const float y = (float)p[r] * d;
+            facc[0][r] = __builtin_fmaf(y, as4[e], facc[0][r]);
+          }
+        }
+      }
+    }
+  };
+  load(st[0], 0);
+  for (int kt = 0; kt < KT; kt += 2) {
+    if (kt + 1 < KT) load(st[1], kt + 1);
+    stage(st[0], kt);
+    if (kt + 1 < KT) {
+      if (kt + 2 < KT) load(st[0], kt + 2);
+      stage(st[1], kt + 1);
+    }
+  }
+  moe_epilogue<GU, NW, 1, 4 * NQ>(facc, tile, a_rows, N, n0, s_rw, s_free, out, out_ld, cmb);
 }
 
 template <bool GU, int NW, int PD, int BM>
@@ -555,13 +679,23 @@ int rk_moe_tile_rows() { return rk_knob("RK_MOE_ROWS", 128) == 64 ? 64 : 128; }
 // registers): 4 waves × 128 columns, weights PD stages ahead, RK_MOE_TILE
 // 0 / 2 / 3 / 4 for PD = 4 / 2 / 3 / 5.
 template <bool GU>
-static hipError_t launch_moe(int tile_rows, const int8_t *A, const float *AS, int as_stride, const int32_t *tok,
+static hipError_t launch_moe(int tile_rows, int max_rows, const int8_t *A, const float *AS, int as_stride, const int32_t *tok,
                              int64_t a_rows,
                              const MoeTile *tiles, int n_tiles, const int8_t *w, const float *ws,
                              int64_t w_stride_e, int64_t ws_stride_e, int ws_stride, int N,
                              int K, const float *row_w, float *out, int out_ld, const MoeCombine &cmb,
                              hipStream_t st) {
   if (n_tiles == 0) return hipSuccess;
+  // RK_MOE_ROWS / RK_MOE_TILE force the ring kernels at any tile size.
+  if (max_rows <= 32 && rk_knob("RK_MOE_ROWS", 0) == 0 && rk_knob("RK_MOE_TILE", -1) < 0) {
+    const int n_col = (N + 127) / 128;
+    MoeCombine c = cmb;
+    c.n_tiles = n_tiles;
+    auto kern = max_rows <= 8 ? moe_few_kernel<GU, 1> : max_rows <= 16 ? moe_few_kernel<GU, 2> : moe_few_kernel<GU, 4>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n_tiles + 7) / 8 * 8 * n_col)), dim3(256), 0, st, A, AS, as_stride, tok,
+                       a_rows, tiles, n_col, w, ws, w_stride_e, ws_stride_e, ws_stride, N, K, row_w, out, out_ld, c);
+    return hipGetLastError();
+  }
 #define RK_MOE_ARGS A, AS, as_stride, tok, a_rows, tiles, n_tiles, w, ws, w_stride_e, ws_stride_e, ws_stride, N, K, \
                     row_w, out, out_ld, cmb, st
   if (tile_rows == 64) {
@@ -582,20 +716,20 @@ static hipError_t launch_moe(int tile_rows, const int8_t *A, const float *AS, in
 #undef RK_MOE_ARGS
 }
 
-hipError_t rk_launch_moe_gemm_gu(int tile_rows, const int8_t *xq, const float *xs, int xs_stride,
+hipError_t rk_launch_moe_gemm_gu(int tile_rows, int max_rows, const int8_t *xq, const float *xs, int xs_stride,
                                  const int32_t *tok, int64_t s, const MoeTile *tiles, int n_tiles, const int8_t *w,
                                  const float *ws, int64_t w_stride_e, int64_t ws_stride_e,
                                  int ws_stride, int N, int K, float *act, hipStream_t st) {
-  return launch_moe<true>(tile_rows, xq, xs, xs_stride, tok, s, tiles, n_tiles, w, ws, w_stride_e, ws_stride_e,
+  return launch_moe<true>(tile_rows, max_rows, xq, xs, xs_stride, tok, s, tiles, n_tiles, w, ws, w_stride_e, ws_stride_e,
                           ws_stride, N, K, nullptr, act, N / 2, MoeCombine{}, st);
 }
 
-hipError_t rk_launch_moe_gemm_down(int tile_rows, const int8_t *aq, const float *as, int as_stride, int64_t rows,
+hipError_t rk_launch_moe_gemm_down(int tile_rows, int max_rows, const int8_t *aq, const float *as, int as_stride, int64_t rows,
                                    const MoeTile *tiles, int n_tiles, const int8_t *w,
                                    const float *ws, int64_t w_stride_e, int64_t ws_stride_e,
                                    int ws_stride, int N, int K, const float *row_w, float *yb,
                                    const MoeCombine &cmb, hipStream_t st) {
-  return launch_moe<false>(tile_rows, aq, as, as_stride, nullptr, rows, tiles, n_tiles, w, ws, w_stride_e, ws_stride_e,
+  return launch_moe<false>(tile_rows, max_rows, aq, as, as_stride, nullptr, rows, tiles, n_tiles, w, ws, w_stride_e, ws_stride_e,
                            ws_stride, N, K, row_w, yb, N, cmb, st);
 }
 
