@@ -2049,7 +2049,8 @@ int moe_experts(rk_weight_id id, const float *x, int64_t s, int top_k, const uin
   // that the host fills them while the GPU works: the rows during the quantizer
   // of x, the slots during gate|up. (With allocations, pageable copies and frees of
   // five lists per call, 8 tokens on 128 experts took 122 us for 78 us of
-  // kernels and 1024 tokens 336 us for 256 us on MI355X; now 100 and 304.)
+  // kernels and 1024 tokens 336 us for 256 us on MI355X; with the lists in one
+  // block 100 and 304, with an upload kernel for the copy commands 280.)
   MoeLists l;
   RK_TRY(moe_lists(*w, s, top_k, ids, &l));
   if (g_eng->moe_pin_bytes < l.bytes) {
@@ -2069,10 +2070,10 @@ int moe_experts(rk_weight_id id, const float *x, int64_t s, int top_k, const uin
     if (part == 0) {
       moe_fill_rows(l, ids, wts, host);
       if (one) moe_fill_slots(l, host);
-      HIP_TRY(hipMemcpyAsync(dev, host, one ? l.bytes : l.slot, hipMemcpyHostToDevice, st), op);
+      HIP_TRY(rk_launch_upload(host, dev, one ? l.bytes : l.slot, st), op);
     } else if (!one) {
       moe_fill_slots(l, host);
-      HIP_TRY(hipMemcpyAsync(dev + l.slot, host + l.slot, l.bytes - l.slot, hipMemcpyHostToDevice, st), op);
+      HIP_TRY(rk_launch_upload(host + l.slot, dev + l.slot, l.bytes - l.slot, st), op);
     }
     return (int)RK_OK;
   });

@@ -72,6 +72,8 @@ bool rk_gemm_f16_skinny(int M, int n, bool glu, int num_cus);
 hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
                                      bool out_f16, int num_cus, hipStream_t st);
 
+// A few KB from page-locked host memory (16-byte aligned, whole 16 bytes).
+hipError_t rk_launch_upload(const void *host, void *dev, size_t bytes, hipStream_t st);
 // Element-wise conversions.
 hipError_t rk_launch_f32_to_f16(const float *x, void *y, int64_t n, hipStream_t st);
 hipError_t rk_launch_f32_to_f16_checked(const float *x, void *y, int64_t n, int *flag, hipStream_t st);

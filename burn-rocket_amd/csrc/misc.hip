@@ -126,6 +126,24 @@ hipError_t rk_launch_f16_to_f32(const void *x, float *y, int64_t n, hipStream_t 
   return hipGetLastError();
 }
 
+// Page-locked host memory (16-byte aligned, bytes a multiple of 16) to the
+// device, read by the kernel itself: for lists of a few KB, where a copy
+// command's own set-up costs more than the transfer (the lists of 1024 tokens on
+// 128 experts, 100 KB: the experts call 304 us with two copies, 280 us so).
+__global__ __launch_bounds__(256) void upload_kernel(const uintx4 *__restrict__ src, uintx4 *__restrict__ dst,
+                                                     int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
+hipError_t rk_launch_upload(const void *host, void *dev, size_t bytes, hipStream_t st) {
+  if (bytes == 0) return hipSuccess;
+  const int64_t n = (int64_t)(bytes / 16);
+  hipLaunchKernelGGL(upload_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const uintx4 *)host,
+                     (uintx4 *)dev, n);
+  return hipGetLastError();
+}
+
 // One workgroup per row. Group maxima are reduced with LDS atomics on the
 // f32 bit pattern (all values are >= 0, so integer order is float order).
 constexpr int QROW_THREADS = 256;
