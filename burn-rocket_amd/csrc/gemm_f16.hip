@@ -315,6 +315,145 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
   }
 }
 
+// The same product with K split over the waves of a workgroup, for grids of at
+// most one tile per CU. There the kernel above is bound by its serial walk: a
+// barrier and an LDS latency per stage, and every fragment read from LDS by
+// two waves. Here each of the NWV waves forms the whole BM×BN tile over every
+// NWV-th stage, in an LDS ring of its own (no barrier in the loop), reads each
+// fragment once, and the partial tiles meet in LDS, added in wave order.
+template <int BM, int BN, int NWV, int ST, int GLU, bool OUT_F16>
+__global__ __launch_bounds__(NWV * 64, 1) void gemm_f16_kwaves_kernel(const f16 *__restrict__ A,
+                                                                      const f16 *__restrict__ B, void *__restrict__ C,
+                                                                      int M, int N, int K, int tiles_m, int tiles_n,
+                                                                      int group_m, int n_out) {
+  constexpr int STAGE = (BM + BN) * ROWB, TM = BM / 16, TN = BN / 16, T = TM * TN;
+  constexpr int A_INS = BM / 8, L = (BM + BN) / 8;  // 8-row copies per stage
+  static_assert(NWV * ST * STAGE <= 160 * 1024 && T * 1024 <= ST * STAGE && (ST - 1) * L <= 63, "geometry");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint8_t *const ring = smem + wave * (ST * STAGE);
+  int tm, tn;
+  tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, group_m, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int KT = (K + KS - 1) / KS;
+  const rsrc_t ra = make_rsrc(A + (size_t)m0 * K, (int64_t)min(M - m0, BM) * K * 2);
+  const rsrc_t rb = make_rsrc(B + (size_t)n0 * K, (int64_t)min(N - n0, BN) * K * 2);
+
+  // Copies and fragment reads: the layout of gemm_f16_kernel.
+  const int crow = lane >> 3, lch = (lane & 7) ^ crow;
+  const uint32_t voff0 = (uint32_t)(crow * K * 2 + lch * 16);
+  auto issue = [&](int slot, int s) {  // stages past the end copy zeros
+    uint8_t *sb = ring + slot * STAGE;
+    const int k0 = s * KS;
+    const uint32_t v0 = k0 + lch * 8 >= K ? OOB_OFFSET : voff0;
+    static_for<L>([&](auto q_c) {
+      constexpr int Q = decltype(q_c)::value;
+      if constexpr (Q < A_INS)
+        bdma16(ra, sb + Q * 1024, v0, (uint32_t)((Q * 8 * K + k0) * 2));
+      else
+        bdma16(rb, sb + Q * 1024, v0, (uint32_t)(((Q - A_INS) * 8 * K + k0) * 2));
+    });
+  };
+  const int frow = lane & 15, ff = frow & 7;
+  const uint32_t off[2] = {(uint32_t)(frow * ROWB + (((lane >> 4) ^ ff) << 4)),
+                           (uint32_t)(frow * ROWB + ((((lane >> 4) + 4) ^ ff) << 4))};
+  floatx4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int i = 0; i < ST; ++i) issue(i, wave + i * NWV);
+  int slot = 0;
+  for (int s = wave; s < KT; s += NWV) {
+    WAIT_VMCNT((ST - 1) * L);  // this stage has landed (later ones may be on their way)
+    asm volatile("" ::: "memory");
+    half8 fa[2][TM], fb[2][TN];
+    const uint8_t *base = ring + slot * STAGE;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[u][i] = *(const half8 *)(base + off[u] + i * 16 * ROWB);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[u][j] = *(const half8 *)(base + off[u] + (BM + j * 16) * ROWB);
+    }
+    WAIT_LGKMCNT0();  // the slot is read: refilled while the MFMAs run
+    asm volatile("" ::: "memory");
+    issue(slot, s + ST * NWV);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[u][j], fa[u][i], acc[i][j], 0, 0, 0);
+    slot = slot + 1 == ST ? 0 : slot + 1;
+  }
+  WAIT_VMCNT(0);  // no copy may still be writing LDS
+
+  floatx4 *mine = (floatx4 *)ring;
+  static_for<T>([&](auto u_c) {
+    constexpr int U = decltype(u_c)::value;
+    mine[U * 64 + lane] = acc[U / TN][U % TN];
+  });
+  __syncthreads();
+  auto tile_sum = [&](int u) {
+    floatx4 v = ((const floatx4 *)smem)[u * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < NWV; ++w) v += ((const floatx4 *)(smem + w * (ST * STAGE)))[u * 64 + lane];
+    return v;
+  };
+  // Four consecutive values of a row of [M, ld], from column n.
+  auto store4 = [&](int m, int n, int ld, const float(&y)[4]) {
+    if (m >= M) return;
+    using E = std::conditional_t<OUT_F16, f16, float>;
+    typedef E E4 __attribute__((ext_vector_type(4)));
+    E *c = (E *)C + (size_t)m * ld + n;
+    if (ld % 4 == 0 && n + 3 < ld) {
+      *(E4 *)c = E4{(E)y[0], (E)y[1], (E)y[2], (E)y[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < ld) c[e] = (E)y[e];
+    }
+  };
+  if constexpr (GLU != 0) {  // tile pairs: gate and up of 16 outputs
+    for (int p = wave; p < T / 2; p += NWV) {
+      const int i = p / (TN / 2), j = p % (TN / 2);
+      const floatx4 g4 = tile_sum(i * TN + 2 * j), u4 = tile_sum(i * TN + 2 * j + 1);
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = glu_apply<GLU>((float)(f16)g4[e], (float)(f16)u4[e]);
+      store4(m0 + i * 16 + frow, n0 / 2 + j * 16 + 4 * (lane >> 4), n_out, y);
+    }
+  } else {
+    for (int u = wave; u < T; u += NWV) {
+      const floatx4 v = tile_sum(u);
+      const float y[4] = {v[0], v[1], v[2], v[3]};
+      store4(m0 + (u / TN) * 16 + frow, n0 + (u % TN) * 16 + 4 * (lane >> 4), N, y);
+    }
+  }
+}
+
+template <int BM, int BN, int NWV, int ST, int GLU = 0, bool OUT_F16 = true>
+static hipError_t launch_kwaves(const f16 *A, const f16 *B, void *C, int M, int N, int K, hipStream_t st,
+                                int n_out = 0) {
+  constexpr int smem = NWV * ST * (BM + BN) * ROWB;
+  auto kern = gemm_f16_kwaves_kernel<BM, BN, NWV, ST, GLU, OUT_F16>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+  hipLaunchKernelGGL(kern, dim3(tm * tn), dim3(NWV * 64), smem, st, A, B, C, M, N, K, tm, tn,
+                     rk_knob("RK_TILE_GROUP_M", 3), n_out);
+  return hipGetLastError();
+}
+
 template <int BM, int BN, int WM, int WN, int ST, int MINW, int GLU = 0, bool OUT_F16 = true>
 static hipError_t launch_gemm_f16(const f16 *A, const f16 *B, void *C, int M, int N, int K,
                                   int ksplit, float *part, unsigned *cnt, hipStream_t st, int n_out = 0) {
@@ -358,6 +497,22 @@ constexpr F16Cfg F16_CFGS[] = {
     {96, 128, 2, .22f},  {256, 192, 1, .42f}, {256, 192, 1, .425f}, {64, 96, 2, .26f},
 };
 constexpr int N_F16_CFGS = sizeof(F16_CFGS) / sizeof(F16_CFGS[0]);
+// Configurations of gemm_f16_kwaves_kernel: 32x32 tiles on 8 waves, 64x32 on 4.
+constexpr int CFG_KW32 = 100, CFG_KW64 = 101;
+// The first of them whose tiles all run at once, one per CU; none otherwise (a
+// second round costs more than the tiled kernel), or for K below 768 (twelve
+// stages: the waves hardly share the walk). MI355X, tiled -> here: 3072->1024
+// 16 rows 11.3 -> 5.8 us, 256 rows (256 tiles of 32x32) 11.7 -> 6.5, 512 rows
+// (256 tiles of 64x32) 12.1 -> 8.8, 700 rows (two rounds) 12.3 -> 16.7;
+// 1024->1024 512 rows 6.1 -> 5.4; 1152->3456 128 rows 6.4 -> 5.5; gate|up
+// 1024->2x3072 32 rows 6.0 -> 4.7, 64 rows 6.1 -> 5.3. 64x64 tiles on 4 or 8
+// waves are slower (3072->1024, 512 rows: 12.1 and 10.5 us).
+int kwaves_cfg(int M, int N, int K, int num_cus) {
+  if (K < 768 || rk_knob("RK_F16_KWAVES", 1) == 0) return -1;
+  const int64_t n32 = (N + 31) / 32;
+  if ((int64_t)((M + 31) / 32) * n32 <= num_cus) return CFG_KW32;
+  return (int64_t)((M + 63) / 64) * n32 <= num_cus ? CFG_KW64 : -1;
+}
 
 hipError_t launch_cfg(int c, const f16 *a, const f16 *b, f16 *d, int M, int N, int K, int ks, float *part,
                       unsigned *cnt, hipStream_t st) {
@@ -426,6 +581,10 @@ F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu) {
   int ks = rk_knob("RK_F16_KSPLIT", 1);
   if (ks > stages) ks = stages;
   F16Plan p;
+  if (!cfg_ok && ks == 1 && kwaves_cfg(M, N, K, num_cus) >= 0) {
+    p.cfg = kwaves_cfg(M, N, K, num_cus);
+    return p;
+  }
   double best = 1e300;
   for (int c = 0; c < N_F16_CFGS; ++c) {
     if (cfg_ok && c != cfg) continue;
@@ -452,6 +611,8 @@ F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu) {
 
 hipError_t rk_launch_gemm_f16(const F16Plan &p, const void *A, const void *B, void *C, int M, int N, int K,
                               float *part, unsigned *cnt, hipStream_t st) {
+  if (p.cfg == CFG_KW32) return launch_kwaves<32, 32, 8, 2>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
+  if (p.cfg == CFG_KW64) return launch_kwaves<64, 32, 4, 3>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
   return launch_cfg(p.cfg, (const f16 *)A, (const f16 *)B, (f16 *)C, M, N, K, p.ksplit, part, cnt, st);
 }
 
@@ -460,6 +621,8 @@ template <int GLU, bool OUT_F16>
 hipError_t launch_glu_cfg(int c, const f16 *a, const f16 *b, void *d, int M, int N, int K, int n_out, int ks,
                           float *part, unsigned *cnt, hipStream_t st) {
   switch (c) {
+    case CFG_KW32: return launch_kwaves<32, 32, 8, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW64: return launch_kwaves<64, 32, 4, 3, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case 0: return launch_gemm_f16<256, 128, 4, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 1: return launch_gemm_f16<192, 192, 2, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 2: return launch_gemm_f16<128, 128, 2, 2, 4, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);

@@ -68,7 +68,7 @@ hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st);
 // N, or n_out of a gate|up product.
 bool rk_gemm_i8_skinny(const I8GemmArgs &g);
 hipError_t rk_launch_gemm_i8_skinny(const I8GemmArgs &g, hipStream_t st);
-bool rk_gemm_f16_skinny(int M, int n, bool glu, int num_cus);
+bool rk_gemm_f16_skinny(int M, int n, int K, bool glu, int num_cus);
 hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
                                      bool out_f16, int num_cus, hipStream_t st);
 

@@ -15,7 +15,7 @@
 //   int8 per token   12 rows, 1024->3072 8.7 -> 4.0;  3072->1024 20.0 -> 7.2;
 //                    256 rows, 3072->1024 20.5 -> 8.8
 //   int8 group 32    16 rows, 1024->3072 11.1 -> 4.4; 256 rows, 3072->1024 28.5 -> 11.4
-//   fp16             1 row, 1024->3072 5.4 -> 3.4;    64 rows, 3072->1024 11.6 -> 7.2
+//   fp16             1 row, 1024->3072 5.4 -> 3.4;    64 rows, 1024->1024 5.8 -> 3.9
 // 16 waves per workgroup gain 0.4 us on K = 3072 and lose as much on K = 1024;
 // int8 workgroups of 64 rows (half the weight reads) are 0.8 to 3.4 us slower.
 #include "common.hpp"
@@ -305,34 +305,39 @@ static hipError_t launch_skinny_f16(const void *A, const void *B, void *C, int M
   return hipGetLastError();
 }
 
-// The smallest tile (1x1, 2x1 or 1x2 of 16x16) that one round of workgroups
-// covers, none if that takes larger ones: 32x32 tiles lose to the tiled kernel
-// (1152->4304, 32 rows: 6.1 us tiled, 6.4 us on 32x32). MI355X, tiled -> here:
-// 1024->4096 32 rows (2x1) 5.7 -> 4.8 us; 1152->4304 16 rows (1x2) 5.9 -> 5.1;
-// 3072->1024 64 rows (1x1) 11.6 -> 7.2, 128 rows (2x1) 11.7 -> 10.0. A gate|up
-// product needs a gate and an up tile per workgroup (1x2): 1024->2x3072 12 rows
-// 5.5 -> 4.6 us, 3072->2x1024 64 rows 11.5 -> 10.1; past one round it loses
-// (1152->2x4304 12 rows, 269 workgroups: 6.0 -> 7.5), and 32x32 tiles lose there
-// too (3072->2x1024 128 rows 11.6 -> 13.0). n: the outputs of one product of a gate|up pair. A tile or split
-// forced by RK_F16_TILE / RK_F16_KSPLIT keeps the tiled kernel.
-static int f16_skinny_tile(int M, int n, bool glu, int num_cus) {
+// n: the outputs of one product of a gate|up pair. Below K = 768: the smallest
+// tile (1x1, 2x1 or 1x2 of 16x16; gate|up needs 1x2) that one round of
+// workgroups covers, none if that takes larger ones. From there
+// gemm_f16_kwaves_kernel shares the reads of a 32x32 tile and these win only
+// with a few rows, or while 1x1 tiles do for a short K (MI355X, here / there:
+// 3072->1024 1 row 5.1 / 5.8 us, 8 rows 6.2 / 5.8, 16 rows 7.2 / 5.8;
+// 2048->1024 8 rows 4.8 / 4.9, 16 rows 5.4 / 5.0; 4304->1152 8 rows 6.3 / 6.9;
+// 1024->1024 64 rows 3.9 / 4.2; 1024->3072 32 rows, 2x1, 4.8 / 4.3; gate|up
+// 1024->2x3072 8 rows 4.5 / 4.7, 16 rows 4.9 / 4.7). A tile or split forced by
+// RK_F16_TILE / RK_F16_KSPLIT keeps the tiled kernel.
+static int f16_skinny_tile(int M, int n, int K, bool glu, int num_cus) {
   if (M > 128) return 0;
   const int64_t m16 = (M + 15) / 16, m32 = (M + 31) / 32, n16 = (n + 15) / 16, n32 = (n + 31) / 32;
+  if (K >= 768) {
+    if (m16 * n16 > num_cus) return 0;
+    if (glu) return K < 1536 && M <= 8 ? 12 : 0;
+    return K < 1536 || M <= 8 ? 11 : 0;
+  }
   if (glu) return m16 * n16 <= num_cus ? 12 : 0;
   if (m16 * n16 <= num_cus) return 11;
   if (m32 * n16 <= num_cus) return 21;
   return m16 * n32 <= num_cus ? 12 : 0;
 }
 
-bool rk_gemm_f16_skinny(int M, int n, bool glu, int num_cus) {
+bool rk_gemm_f16_skinny(int M, int n, int K, bool glu, int num_cus) {
   if (rk_knob("RK_SKINNY", 1) == 0 || rk_knob("RK_F16_TILE", -1) >= 0 || rk_knob("RK_F16_KSPLIT", 1) != 1) return false;
-  return f16_skinny_tile(M, n, glu, num_cus) != 0;
+  return f16_skinny_tile(M, n, K, glu, num_cus) != 0;
 }
 
 hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
                                      bool out_f16, int num_cus, hipStream_t st) {
   if (!glu) n_out = N, out_f16 = true;
-  switch (f16_skinny_tile(M, n_out, glu != 0, num_cus)) {
+  switch (f16_skinny_tile(M, n_out, K, glu != 0, num_cus)) {
     case 11: return launch_skinny_f16<1, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
     case 21: return launch_skinny_f16<2, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
     case 12: return launch_skinny_f16<1, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);

@@ -55,7 +55,7 @@ def test_skinny_i8(rk, orc, m, k, n, group):
             close(got, ref, f16)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 8, 1), (16, 72, 16), (17, 1152, 33), (32, 1016, 200), (5, 3072, 96),
+@pytest.mark.parametrize("m,k,n", [(1, 8, 1), (16, 72, 16), (17, 1152, 33), (32, 1016, 200), (5, 3072, 96), (48, 704, 1400),
                                    (40, 96, 1500), (20, 192, 4200), (12, 136, 4300), (128, 200, 1000)])
 def test_skinny_f16(rk, orc, m, k, n):
     note(f"skinny fp16 m={m} k={k} n={n}")
@@ -69,8 +69,51 @@ def test_skinny_f16(rk, orc, m, k, n):
           (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32), True)
 
 
+# K split over the waves of 32x32 tiles (8 waves) and 64x32 tiles (4 waves): one
+# row, tile edges, K of less than two stages per wave and one that ends inside
+# a stage, odd N, and the largest grids of either tile.
+@pytest.mark.parametrize("m,k,n", [(9, 1536, 1), (33, 768, 1050), (64, 1544, 3000), (255, 776, 1000), (300, 1160, 800),
+                                   (512, 3072, 1024), (65, 4304, 2001)])
+def test_kwaves_f16(rk, orc, m, k, n):
+    note(f"fp16 K over waves m={m} k={k} n={n}")
+    r = np.random.default_rng(m + k + n)
+    a = r.standard_normal((m, k)).astype(np.float16)
+    b = (r.standard_normal((n, k)) * 0.05).astype(np.float16)
+    da, dc = dev(rk, a.view(np.uint16)), rk.DeviceBuffer(m * n * 2)
+    wid = rk.pack(b)
+    ref = (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32)
+    for _ in range(2):  # the sums have one order
+        assert rk.lib().rk_matmul_f16_dev(int(wid), da.ptr, m, k, dc.ptr, None) == 0, rk.lib().rk_last_error()
+        rk.synchronize()
+        got = dc.download((m, n), np.uint16).view(np.float16).astype(np.float32)
+        close(got, ref, True)
+
+
 @pytest.mark.parametrize("glu", ["silu", "gelu"])
-@pytest.mark.parametrize("m,k,n", [(1, 64, 3), (16, 1152, 40), (32, 416, 64), (29, 3072, 17),
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("m,k,n", [(9, 1536, 5), (40, 776, 1900), (64, 1160, 1900), (130, 3072, 300)])
+def test_kwaves_f16_glu(rk, orc, m, k, n, glu, f16):
+    """gate|up against the glue of float64 products rounded to fp16: a product next to a rounding
+    midpoint may round the other way (one fp16 step of the gate or up value)."""
+    note(f"fp16 gate|up K over waves m={m} k={k} n={n} {glu} f16={f16}")
+    r = np.random.default_rng(m + k + n)
+    x = r.standard_normal((m, k)).astype(np.float16)
+    w = [(r.standard_normal((n, k)) * 0.05).astype(np.float16) for _ in range(2)]
+    dx, dy = dev(rk, x.view(np.uint16)), rk.DeviceBuffer(m * n * 4)
+    kind, glue = (rk.GLU_SILU, orc.silu_mul) if glu == "silu" else (rk.GLU_GELU, orc.gelu_mul)
+    wid = rk.pack_f16_glu(*[t.astype(np.float32) for t in w])
+    assert rk.lib().rk_matmul_f16_glu_dev(int(wid), dx.ptr, m, k, kind, dy.ptr, int(f16), None) == 0
+    rk.synchronize()
+    got = dy.download((m, n), np.uint16).view(np.float16).astype(np.float32) if f16 else dy.download((m, n), np.float32)
+    g, u = [(x.astype(np.float64) @ t.astype(np.float64).T).astype(np.float16).astype(np.float32) for t in w]
+    ref = glue(g, u)
+    # |d silu| and |d gelu| <= 1.13; a step is 2^-10 of the value; an fp16 result rounds once more
+    step = 2.0 ** -10 * 1.13 * (np.abs(g) * np.abs(u) + np.abs(g * u)) + 1e-5
+    assert (np.abs(got - ref) <= step + (2.0 ** -10 * np.abs(ref) if f16 else 0)).all()
+
+
+@pytest.mark.parametrize("glu", ["silu", "gelu"])
+@pytest.mark.parametrize("m,k,n", [(1, 64, 3), (8, 1152, 40), (32, 416, 64), (29, 3072, 17),
                                    (24, 128, 1500), (128, 256, 72), (9, 96, 4000)])
 def test_skinny_glu_equals_products_then_glue(rk, orc, m, k, n, glu):
     """The fused forms give what the two plain products and the glue op give, bit for bit."""
