@@ -487,9 +487,10 @@ namespace {
 struct F16Cfg {
   int bm, bn, per_cu;
   float eff;
+  float eff_alone = 0;  // of a tile alone on its CU where two fit, when it differs
 };
 constexpr F16Cfg F16_CFGS[] = {
-    {256, 128, 1, .40f}, {192, 192, 1, .38f}, {128, 128, 1, .32f}, {128, 64, 2, .26f},
+    {256, 128, 1, .40f}, {192, 192, 1, .38f}, {128, 128, 1, .32f}, {128, 64, 2, .26f, .29f},
     {64, 64, 2, .27f},   {128, 256, 1, .41f}, {96, 128, 1, .27f},  {128, 192, 1, .34f},
     {192, 128, 1, .35f}, {64, 128, 2, .25f},  {192, 192, 1, .41f}, {192, 192, 1, .42f},
     {128, 128, 1, .33f}, {128, 192, 1, .36f}, {192, 128, 1, .42f}, {128, 192, 2, .36f},
@@ -566,7 +567,11 @@ double cfg_time(int c, int ks, int M, int N, int K, int num_cus) {
   const long slots = (long)num_cus * f.per_cu;
   const long rounds = (wgs + slots - 1) / slots;
   const long held = std::min<long>(f.per_cu, (wgs + num_cus - 1) / num_cus);
-  double t = rounds * (3e-6 + held * 2.0 * f.bm * f.bn * ((double)K / ks) / (9.83e12 * f.eff));
+  // (128x64 tiles, one per CU, priced like two per CU lost to 64x64 tiles:
+  // 1024->4096 512 rows 12.4 -> 8.6 us, 3072->1024 2000 rows 23.3 -> 20.8,
+  // gate|up 3072->2x1024 1000 rows 25.5 -> 22.1, MI355X)
+  const float eff = held == 1 && f.eff_alone > 0 ? f.eff_alone : f.eff;
+  double t = rounds * (3e-6 + held * 2.0 * f.bm * f.bn * ((double)K / ks) / (9.83e12 * eff));
   if (ks > 1) t += 1e-6 + (double)wgs * f.bm * f.bn * 4 * 2 / 10e12;
   return t;
 }
