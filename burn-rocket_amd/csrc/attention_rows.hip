@@ -443,11 +443,14 @@ hipError_t launch_rows_d(const AttnArgs &a, const void *v, int64_t v_ts, int64_t
 // tiles) 61.9 -> 44.8, 1024 queries (192 tiles) 62 -> 75. A tile height or split
 // forced by RK_ATTN_ROWS / RK_ATTN_SPLIT / RK_ATTN_SPLIT_TILES keeps
 // attn_fa_kernel; RK_ATTN_FEW=0 turns this kernel off.
-bool rk_attn_rows_fits(const AttnArgs &a, int64_t v_tok_stride) {
+bool rk_attn_rows_fits(const AttnArgs &a, const void *v, int64_t v_tok_stride) {
   if (a.n_kv_heads <= 0 || a.n_head % a.n_kv_heads) return false;
   if (rk_knob("RK_ATTN_FEW", 1) == 0 || rk_knob("RK_ATTN_SPLIT", 0) != 0 || rk_knob("RK_ATTN_ROWS", 0) != 0 ||
       rk_knob("RK_ATTN_SPLIT_TILES", -1) >= 0)
     return false;
+  // V is copied to LDS in 16-byte pieces, which attn_fa_kernel's own transposing
+  // launch does not need to be aligned.
+  if (((uintptr_t)v & 15) != 0 || v_tok_stride % 8 != 0) return false;
   // K and V of one kv head are addressed with 32-bit byte offsets.
   const int64_t reach = (int64_t)1 << 31, keys = (int64_t)a.n_kv + CK;
   if (keys * a.k_tok_stride * 2 >= reach || keys * v_tok_stride * 2 >= reach) return false;

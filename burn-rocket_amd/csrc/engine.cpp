@@ -1264,7 +1264,7 @@ int attn_workspace(CallScope &cs, size_t part_bytes, size_t n_cnt, AttnArgs &a, 
 
 // Few query rows: V is read as it lies, no Vᵀ. *done: whether the call was one.
 int attn_rows_run(CallScope &cs, AttnArgs a, const void *v, int64_t v_ts, bool *done, const char *op) {
-  *done = rk_attn_rows_fits(a, v_ts);
+  *done = rk_attn_rows_fits(a, v, v_ts);
   if (!*done) return RK_OK;
   size_t part_bytes, n_cnt;
   rk_attn_rows_workspace(a, &part_bytes, &n_cnt);
@@ -2400,7 +2400,7 @@ extern "C" int rk_attention_qkv_dev(void *qkv, int64_t s, int64_t row_stride, in
   const uint16_t *kp = (const uint16_t *)qkv + (int64_t)n_head * head_dim, *vp = kp + (int64_t)n_kv_heads * head_dim;
   const AttnArgs rows = attn_args(qkv, kp, out, s, s, n_head, n_kv_heads, head_dim, scale, softcap, mode, window, q0, k0,
                                   false, row_stride, row_stride, out_stride);
-  if (rk_attn_rows_fits(rows, row_stride)) {
+  if (rk_attn_rows_fits(rows, vp, row_stride)) {
     HIP_TRY(rk_launch_qk_norm_rope(qkv, row_stride, (int)s, n_head, n_kv_heads, head_dim, q_norm_w, k_norm_w,
                                    (float)eps, cos, sin, cs_dtype, RK_DTYPE_F16, st), name);
     bool done;

@@ -200,7 +200,7 @@ long rk_attn_split_floats(int head_dim);
 // as it lies (a.vt is not used): whether a call goes there; its workspace (a.part
 // of part_bytes and a.cnt of n_cnt counters that start at zero and are left at
 // zero; both may be 0); the launch.
-bool rk_attn_rows_fits(const AttnArgs &a, int64_t v_tok_stride);
+bool rk_attn_rows_fits(const AttnArgs &a, const void *v, int64_t v_tok_stride);
 void rk_attn_rows_workspace(const AttnArgs &a, size_t *part_bytes, size_t *n_cnt);
 hipError_t rk_launch_attention_rows(const AttnArgs &a, const void *v, int64_t v_tok_stride, int64_t v_head_stride,
                                     hipStream_t st);

@@ -71,3 +71,18 @@ def test_rows_large_scores(rk, orc):
     q, k, v = data(7, 1, n_kv, h, kv, d)
     k = (k * np.linspace(0.1, 6, n_kv)[:, None]).astype(np.float16)
     check(orc, run(rk, q, k, v, h, kv, d, 1.0), orc.attention_ref(q, k, v, h, kv, d, 1.0))
+
+
+def test_rows_unaligned_v_keeps_its_kernel(rk, orc):
+    """V at an address that is not a multiple of 16 bytes goes to the kernel that takes it."""
+    note("rows attention, V 4 bytes off")
+    h, kv, d, n_q, n_kv = 4, 2, 64, 3, 200
+    q, k, v = data(5, n_q, n_kv, h, kv, d)
+    b = [rk.DeviceBuffer.from_array(t.view(np.uint16)) for t in (q, k)]
+    dv = rk.DeviceBuffer.from_array(np.concatenate([np.zeros(2, np.uint16), v.view(np.uint16).reshape(-1)]))
+    o = rk.DeviceBuffer(n_q * h * d * 2)
+    assert rk.lib().rk_attention_dev(b[0].ptr, b[1].ptr, dv.ptr + 4, n_q, n_kv, h, kv, d, 0.125, 0.0, 0, -1, 0, 0,
+                                     o.ptr, None) == 0, rk.lib().rk_last_error()
+    rk.synchronize()
+    check(orc, o.download((n_q, h * d), np.uint16).view(np.float16).astype(np.float32),
+          orc.attention_ref(q, k, v, h, kv, d, 0.125))
