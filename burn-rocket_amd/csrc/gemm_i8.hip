@@ -762,7 +762,10 @@ __global__ __launch_bounds__(KG *WM *WN * 64, MINW) void gemm_i8_q8_kernel(
           if constexpr (MODE == MODE_RAW) {
             __builtin_nontemporal_store(iacc[i][j][r], (int32_t *)Cout + (size_t)m * N + n);
           } else {
-            const float v = GROUPED ? facc[i][j][r] : as4[r >> 2][r & 3] * facc[i][j][r];
+            float v = GROUPED ? facc[i][j][r] : as4[r >> 2][r & 3] * facc[i][j][r];
+            // the f32 sum is rounded to fp16: left alone, the compiler folds the
+            // last FMA into the conversion in some forms and rounds once
+            if constexpr (GROUPED && OUT_F16) asm("" : "+v"(v));
             if constexpr (OUT_F16)
               ((f16 *)Cout)[(size_t)m * N + n] = (f16)v;
             else  // 32 lanes fill one 128-byte line of a row: streamed past L2

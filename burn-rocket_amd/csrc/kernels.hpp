@@ -64,7 +64,7 @@ struct I8GemmArgs {
 };
 hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st);
 // GEMMs with few output tiles (skinny.hip): whether a launch goes there, and
-// the launches. fp16: C [M, N] fp16, or with glu the gate|up forms above; n is
+// the launches. int8: the bits of rk_launch_gemm_i8's own kernels. fp16: C [M, N] fp16, or with glu the gate|up forms above; n is
 // N, or n_out of a gate|up product.
 bool rk_gemm_i8_skinny(const I8GemmArgs &g);
 hipError_t rk_launch_gemm_i8_skinny(const I8GemmArgs &g, hipStream_t st);
