@@ -825,12 +825,13 @@ int launch_i8(const Weight &w, const int8_t *a, const float *as, int as_stride, 
 // zeroed when first allocated (every launch leaves them at zero).
 int gemm_f16_run(CallScope &cs, const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k,
                  const char *op, int glu = 0, int64_t n_out = 0, bool out_f16 = true) {
-  if (rk_gemm_f16_skinny((int)m, (int)(glu ? n_out : n), (int)k, glu != 0, g_eng->num_cus)) {
+  const int n1 = (int)(glu ? n_out : n), kwaves = rk_gemm_f16_kwaves((int)m, n1, (int)k, g_eng->num_cus);
+  if (rk_gemm_f16_skinny(kwaves, (int)m, n1, (int)k, glu != 0, g_eng->num_cus)) {
     HIP_TRY(rk_launch_gemm_f16_skinny(a, b, c, (int)m, (int)n, (int)k, glu, (int)n_out, out_f16, g_eng->num_cus, cs.st),
             op);
     return RK_OK;
   }
-  const F16Plan p = rk_gemm_f16_plan((int)m, (int)n, (int)k, g_eng->num_cus, glu != 0);
+  const F16Plan p = rk_gemm_f16_plan((int)m, (int)n, (int)k, g_eng->num_cus, glu != 0, kwaves);
   float *part = nullptr;
   unsigned *cnt = nullptr;
   if (p.ksplit > 1) {

@@ -498,21 +498,21 @@ constexpr F16Cfg F16_CFGS[] = {
     {96, 128, 2, .22f},  {256, 192, 1, .42f}, {256, 192, 1, .425f}, {64, 96, 2, .26f},
 };
 constexpr int N_F16_CFGS = sizeof(F16_CFGS) / sizeof(F16_CFGS[0]);
-// Configurations of gemm_f16_kwaves_kernel: 32x32 tiles on 8 waves, 64x32 on 4.
-constexpr int CFG_KW32 = 100, CFG_KW64 = 101;
-// The first of them whose tiles all run at once, one per CU; none otherwise (a
-// second round costs more than the tiled kernel), or for K below 768 (twelve
-// stages: the waves hardly share the walk). MI355X, tiled -> here: 3072->1024
-// 16 rows 11.3 -> 5.8 us, 256 rows (256 tiles of 32x32) 11.7 -> 6.5, 512 rows
-// (256 tiles of 64x32) 12.1 -> 8.8, 700 rows (two rounds) 12.3 -> 16.7;
-// 1024->1024 512 rows 6.1 -> 5.4; 1152->3456 128 rows 6.4 -> 5.5; gate|up
-// 1024->2x3072 32 rows 6.0 -> 4.7, 64 rows 6.1 -> 5.3. 64x64 tiles on 4 or 8
-// waves are slower (3072->1024, 512 rows: 12.1 and 10.5 us).
-int kwaves_cfg(int M, int N, int K, int num_cus) {
-  if (K < 768 || rk_knob("RK_F16_KWAVES", 1) == 0) return -1;
-  const int64_t n32 = (N + 31) / 32;
-  if ((int64_t)((M + 31) / 32) * n32 <= num_cus) return CFG_KW32;
-  return (int64_t)((M + 63) / 64) * n32 <= num_cus ? CFG_KW64 : -1;
+// Configurations of gemm_f16_kwaves_kernel, by the waves K is split over: 32x32
+// tiles on 8, 64x32 on 4, one per CU. A gate|up product has twice the tiles of the
+// plain product whose split it takes: where those are more than one round, larger
+// tiles with fewer stages in flight, or for a short K on 4 waves several
+// workgroups per CU (MI355X, us: 8 waves, 1024->2x1024 256 rows 64x32 tiles 5.5,
+// 32x32 two per CU 6.1; 3072->2x1024 200 rows 64x32 8.7, 32x64 11.8; 4 waves,
+// 1024->2x3072 128 rows 64x32 6.7, 64x64 7.5; 2048->2x1024 512 rows 64x64 10.1,
+// 64x32 11.2).
+constexpr int CFG_KW8 = 100, CFG_KW4 = 101, CFG_KW8_64x32 = 102, CFG_KW8_32x64 = 103, CFG_KW4_SHORT = 104,
+              CFG_KW4_64x64 = 105;
+int kwaves_cfg(int kwaves, int M, int N, int K, bool glu, int num_cus) {
+  const int64_t n32 = (N + 31) / 32, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
+  if (!glu || (kwaves == 8 ? m32 : m64) * n32 <= num_cus) return kwaves == 8 ? CFG_KW8 : CFG_KW4;
+  if (kwaves == 8) return m64 * n32 <= num_cus ? CFG_KW8_64x32 : CFG_KW8_32x64;
+  return K < 1536 ? CFG_KW4_SHORT : CFG_KW4_64x64;
 }
 
 hipError_t launch_cfg(int c, const f16 *a, const f16 *b, f16 *d, int M, int N, int K, int ks, float *part,
@@ -577,7 +577,29 @@ double cfg_time(int c, int ks, int M, int N, int K, int num_cus) {
 }
 }  // namespace
 
-F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu) {
+// Eight or four waves while the plain product's 32x32 or 64x32 tiles all run at
+// once, one per CU (a second round costs more than the tiled kernel); below K = 768
+// (twelve stages: the waves hardly share the walk) eight on the 16-row tiles of
+// skinny.hip. MI355X, tiled -> split: 3072->1024 16 rows 11.3 -> 5.8 us, 256 rows
+// (256 tiles of 32x32) 11.7 -> 6.5, 512 rows (256 tiles of 64x32) 12.1 -> 8.8, 700
+// rows (two rounds) 12.3 -> 16.7; 1024->1024 512 rows 6.1 -> 5.4; 1152->3456 128
+// rows 6.4 -> 5.5; gate|up 1024->2x3072 32 rows 6.0 -> 4.7, 64 rows 6.1 -> 5.3. 64x64
+// tiles of a plain product are slower (3072->1024, 512 rows: 12.1 and 10.5 us on 4
+// and 8 waves). The fused form takes the plain one's split although it has twice
+// the tiles: with a split of its own it would differ from the plain products by
+// their rounding. At the upper end that costs a tenth (1024->2x1024 512 rows 6.4 us
+// unsplit, 6.9 on four waves; 2048->2x1024 9.2 and 10.1).
+int rk_gemm_f16_kwaves(int M, int n, int K, int num_cus) {
+  if (rk_knob("RK_F16_TILE", -1) >= 0 || rk_knob("RK_F16_KSPLIT", 1) != 1) return 1;
+  const bool skinny = rk_knob("RK_SKINNY", 1) != 0;
+  const int64_t m16 = (M + 15) / 16, m32 = (M + 31) / 32, m64 = (M + 63) / 64, n16 = (n + 15) / 16, n32 = (n + 31) / 32;
+  if (K < 768)
+    return skinny && M <= 128 && std::min({m16 * n16, m32 * n16, m16 * n32}) <= num_cus ? 8 : 1;
+  if (rk_knob("RK_F16_KWAVES", 1) == 0) return skinny && M <= 128 && m16 * n16 <= num_cus && (K < 1536 || M <= 8) ? 8 : 1;
+  return m32 * n32 <= num_cus ? 8 : m64 * n32 <= num_cus ? 4 : 1;
+}
+
+F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu, int kwaves) {
   const int stages = (K + KS - 1) / KS;
   int cfg = rk_knob("RK_F16_TILE", -1);
   const bool cfg_ok = cfg >= 0 && cfg < N_F16_CFGS &&
@@ -586,8 +608,8 @@ F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu) {
   int ks = rk_knob("RK_F16_KSPLIT", 1);
   if (ks > stages) ks = stages;
   F16Plan p;
-  if (!cfg_ok && ks == 1 && kwaves_cfg(M, N, K, num_cus) >= 0) {
-    p.cfg = kwaves_cfg(M, N, K, num_cus);
+  if (kwaves > 1) {
+    p.cfg = kwaves_cfg(kwaves, M, N, K, glu, num_cus);
     return p;
   }
   double best = 1e300;
@@ -616,8 +638,8 @@ F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu) {
 
 hipError_t rk_launch_gemm_f16(const F16Plan &p, const void *A, const void *B, void *C, int M, int N, int K,
                               float *part, unsigned *cnt, hipStream_t st) {
-  if (p.cfg == CFG_KW32) return launch_kwaves<32, 32, 8, 2>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
-  if (p.cfg == CFG_KW64) return launch_kwaves<64, 32, 4, 3>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
+  if (p.cfg == CFG_KW8) return launch_kwaves<32, 32, 8, 2>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
+  if (p.cfg == CFG_KW4) return launch_kwaves<64, 32, 4, 3>((const f16 *)A, (const f16 *)B, C, M, N, K, st);
   return launch_cfg(p.cfg, (const f16 *)A, (const f16 *)B, (f16 *)C, M, N, K, p.ksplit, part, cnt, st);
 }
 
@@ -626,8 +648,12 @@ template <int GLU, bool OUT_F16>
 hipError_t launch_glu_cfg(int c, const f16 *a, const f16 *b, void *d, int M, int N, int K, int n_out, int ks,
                           float *part, unsigned *cnt, hipStream_t st) {
   switch (c) {
-    case CFG_KW32: return launch_kwaves<32, 32, 8, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
-    case CFG_KW64: return launch_kwaves<64, 32, 4, 3, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW8: return launch_kwaves<32, 32, 8, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW4: return launch_kwaves<64, 32, 4, 3, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW8_64x32: return launch_kwaves<64, 32, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW8_32x64: return launch_kwaves<32, 64, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW4_SHORT: return launch_kwaves<64, 32, 4, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_KW4_64x64: return launch_kwaves<64, 64, 4, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case 0: return launch_gemm_f16<256, 128, 4, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 1: return launch_gemm_f16<192, 192, 2, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 2: return launch_gemm_f16<128, 128, 2, 2, 4, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);

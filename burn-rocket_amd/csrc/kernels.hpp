@@ -23,7 +23,11 @@ struct F16Plan {
   int64_t part_floats = 0;
   int64_t n_cnt = 0;
 };
-F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu);
+// The waves of a workgroup that K is split over in a product of n outputs (1: not
+// split): of the product's shape alone, the same for a plain product and for the
+// two of a gate|up pair, so that both forms sum in the same order.
+int rk_gemm_f16_kwaves(int M, int n, int K, int num_cus);
+F16Plan rk_gemm_f16_plan(int M, int N, int K, int num_cus, bool glu, int kwaves);
 // fp16 GEMM, C[M,N] = A[M,K]·B[N,K]ᵀ, K % 8 == 0.
 hipError_t rk_launch_gemm_f16(const F16Plan &p, const void *A, const void *B, void *C, int M, int N, int K,
                               float *part, unsigned *cnt, hipStream_t st);
@@ -31,7 +35,7 @@ hipError_t rk_launch_gemm_f16(const F16Plan &p, const void *A, const void *B, vo
 // fp16 GEMM with a gate|up glue epilogue: B [N, K] holds gate and up rows
 // interleaved per 16 (N = 32·ceil(n_out/16)); C [M, n_out] = glue(gate·a,
 // up·a) with both products rounded to fp16 first; glu 1 silu·up, 2 gelu·up;
-// C f32 or (out_f16) fp16. p from rk_gemm_f16_plan(.., glu = true).
+// C f32 or (out_f16) fp16. p from rk_gemm_f16_plan(.., glu = true, ..).
 hipError_t rk_launch_gemm_f16_glu(const F16Plan &p, const void *A, const void *B, void *C, int M, int N, int K,
                                   int n_out, int glu, bool out_f16, float *part, unsigned *cnt, hipStream_t st);
 // Element type conversion (RK_DTYPE_* src → dst), round to nearest even.
@@ -64,11 +68,12 @@ struct I8GemmArgs {
 };
 hipError_t rk_launch_gemm_i8(const I8GemmArgs &g, hipStream_t st);
 // GEMMs with few output tiles (skinny.hip): whether a launch goes there, and
-// the launches. int8: the bits of rk_launch_gemm_i8's own kernels. fp16: C [M, N] fp16, or with glu the gate|up forms above; n is
-// N, or n_out of a gate|up product.
+// the launches. int8: the bits of rk_launch_gemm_i8's own kernels. fp16 (K split over
+// `kwaves` waves): C [M, N] fp16, or with glu the gate|up forms above; n is N, or
+// n_out of a gate|up product.
 bool rk_gemm_i8_skinny(const I8GemmArgs &g);
 hipError_t rk_launch_gemm_i8_skinny(const I8GemmArgs &g, hipStream_t st);
-bool rk_gemm_f16_skinny(int M, int n, int K, bool glu, int num_cus);
+bool rk_gemm_f16_skinny(int kwaves, int M, int n, int K, bool glu, int num_cus);
 hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
                                      bool out_f16, int num_cus, hipStream_t st);
 

@@ -570,13 +570,14 @@ __global__ __launch_bounds__(SNW * 64, 2) void skinny_f16_kernel(const f16 *__re
     for (int w = 1; w < SNW; ++w) v += red[(w * T + t) * 256 + e];
     return v;
   };
-  if (glu != GLU_NONE) {
-    for (int x = threadIdx.x; x < TM * 256; x += SNW * 64) {
-      const int i = x >> 8, c = x & 15, r = (x >> 4) & 15;  // columns fastest: coalesced stores
+  if (glu != GLU_NONE) {  // tile pairs: gate and up of 16 outputs
+    for (int x = threadIdx.x; x < T * 128; x += SNW * 64) {
+      const int p = x >> 8, i = p / (TN / 2 ? TN / 2 : 1), j = p % (TN / 2 ? TN / 2 : 1);
+      const int c = x & 15, r = (x >> 4) & 15;  // columns fastest: coalesced stores
       const int e = (c >> 2) * 64 + r * 4 + (c & 3);
-      const int m = m0 + i * 16 + r, oc = n0 / 2 + c;
+      const int m = m0 + i * 16 + r, oc = n0 / 2 + j * 16 + c;
       if (m < M && oc < n_out) {
-        const float g = (float)(f16)value(i * TN, e), u = (float)(f16)value(i * TN + TN - 1, e);
+        const float g = (float)(f16)value(i * TN + 2 * j, e), u = (float)(f16)value(i * TN + 2 * j + 1, e);
         const float y = glu_any(glu, g, u);
         if (out_f16)
           ((f16 *)C)[(size_t)m * n_out + oc] = (f16)y;
@@ -601,42 +602,40 @@ static hipError_t launch_skinny_f16(const void *A, const void *B, void *C, int M
   return hipGetLastError();
 }
 
-// n: the outputs of one product of a gate|up pair. Below K = 768: the smallest
-// tile (1x1, 2x1 or 1x2 of 16x16; gate|up needs 1x2) that one round of
-// workgroups covers, none if that takes larger ones. From there
-// gemm_f16_kwaves_kernel shares the reads of a 32x32 tile and these win only
-// with a few rows, or while 1x1 tiles do for a short K (MI355X, here / there:
-// 3072->1024 1 row 5.1 / 5.8 us, 8 rows 6.2 / 5.8, 16 rows 7.2 / 5.8;
+// Of a product whose K is split over eight waves (rk_gemm_f16_kwaves). n: the outputs
+// of one product of a gate|up pair, whose tiles are twice as wide. Below K = 768:
+// the smallest tile (1x1, 2x1 or 1x2 of 16x16) that one round of workgroups
+// covers. From there gemm_f16_kwaves_kernel shares the reads of a 32x32 tile and
+// these win only with a few rows, or while 1x1 tiles do for a short K (MI355X, here
+// / there: 3072->1024 1 row 5.1 / 5.8 us, 8 rows 6.2 / 5.8, 16 rows 7.2 / 5.8;
 // 2048->1024 8 rows 4.8 / 4.9, 16 rows 5.4 / 5.0; 4304->1152 8 rows 6.3 / 6.9;
 // 1024->1024 64 rows 3.9 / 4.2; 1024->3072 32 rows, 2x1, 4.8 / 4.3; gate|up
-// 1024->2x3072 8 rows 4.5 / 4.7, 16 rows 4.9 / 4.7). A tile or split forced by
-// RK_F16_TILE / RK_F16_KSPLIT keeps the tiled kernel.
+// 1024->2x3072 8 rows 4.5 / 4.7, 16 rows 4.9 / 4.7).
 static int f16_skinny_tile(int M, int n, int K, bool glu, int num_cus) {
-  if (M > 128) return 0;
-  const int64_t m16 = (M + 15) / 16, m32 = (M + 31) / 32, n16 = (n + 15) / 16, n32 = (n + 31) / 32;
+  const int64_t m16 = (M + 15) / 16, m32 = (M + 31) / 32, n16 = (n + 15) / 16;
   if (K >= 768) {
-    if (m16 * n16 > num_cus) return 0;
-    if (glu) return K < 1536 && M <= 8 ? 12 : 0;
-    return K < 1536 || M <= 8 ? 11 : 0;
+    const bool few = glu ? K < 1536 && M <= 8 : K < 1536 || M <= 8;
+    return few && M <= 128 && m16 * n16 <= num_cus ? 11 : 0;
   }
-  if (glu) return m16 * n16 <= num_cus ? 12 : 0;
-  if (m16 * n16 <= num_cus) return 11;
-  if (m32 * n16 <= num_cus) return 21;
-  return m16 * n32 <= num_cus ? 12 : 0;
+  return m16 * n16 <= num_cus ? 11 : m32 * n16 <= num_cus ? 21 : 12;
 }
 
-bool rk_gemm_f16_skinny(int M, int n, int K, bool glu, int num_cus) {
-  if (rk_knob("RK_SKINNY", 1) == 0 || rk_knob("RK_F16_TILE", -1) >= 0 || rk_knob("RK_F16_KSPLIT", 1) != 1) return false;
-  return f16_skinny_tile(M, n, K, glu, num_cus) != 0;
+bool rk_gemm_f16_skinny(int kwaves, int M, int n, int K, bool glu, int num_cus) {
+  return kwaves == 8 && rk_knob("RK_SKINNY", 1) != 0 && f16_skinny_tile(M, n, K, glu, num_cus) != 0;
 }
 
 hipError_t rk_launch_gemm_f16_skinny(const void *A, const void *B, void *C, int M, int N, int K, int glu, int n_out,
                                      bool out_f16, int num_cus, hipStream_t st) {
   if (!glu) n_out = N, out_f16 = true;
-  switch (f16_skinny_tile(M, n_out, K, glu != 0, num_cus)) {
-    case 11: return launch_skinny_f16<1, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
-    case 21: return launch_skinny_f16<2, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
-    case 12: return launch_skinny_f16<1, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+  const int tile = f16_skinny_tile(M, n_out, K, glu != 0, num_cus);
+  if (glu) {
+    if (tile == 11) return launch_skinny_f16<1, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    if (tile == 21) return launch_skinny_f16<2, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    if (tile == 12) return launch_skinny_f16<1, 4>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+  } else {
+    if (tile == 11) return launch_skinny_f16<1, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    if (tile == 21) return launch_skinny_f16<2, 1>(A, B, C, M, N, K, out_f16, glu, n_out, st);
+    if (tile == 12) return launch_skinny_f16<1, 2>(A, B, C, M, N, K, out_f16, glu, n_out, st);
   }
   return hipErrorInvalidValue;
 }

@@ -1,5 +1,6 @@
-"""The order of the sums of the scaled int8 products (groups ascending, whatever kernel a
-call's size takes), through the C ABI: rows that do not depend on the batch they come in."""
+"""The order of the sums: of the scaled int8 products (groups ascending, whatever kernel a
+call's size takes: rows do not depend on the batch they come in), and of fused against plain
+products, through the C ABI."""
 import sys
 
 import numpy as np
@@ -95,3 +96,34 @@ def test_int8_gate_up_equals_products_then_glue(rk, orc, monkeypatch, m, k, n):
             half.append(dy.download((m, n), np.uint16))
         monkeypatch.delenv("RK_SKINNY")
         assert (half[0] == half[1]).all()
+
+
+# K below 768 in each tile the few-tile kernel has; from there one row tile, tiles as wide
+# as a plain product's and twice as wide, K over eight waves, over four and unsplit.
+@pytest.mark.parametrize("m,k,n", [(24, 128, 1500), (40, 96, 1500), (20, 192, 4200), (12, 136, 4300), (8, 1024, 3072),
+                                   (33, 1024, 3072), (64, 1024, 3072), (128, 1024, 3072), (256, 776, 1000),
+                                   (100, 1160, 1900), (70, 776, 3001), (500, 1160, 1000), (300, 1024, 3072)])
+def test_fp16_gate_up_equals_products_then_glue(rk, orc, m, k, n):
+    note(f"fp16 gate|up m={m} k={k} n={n}")
+    lib, r = rk.lib(), np.random.default_rng(m + k + n)
+    x = r.standard_normal((m, k)).astype(np.float16)
+    w = [(r.standard_normal((n, k)) * 0.05).astype(np.float32) for _ in range(2)]
+    dx, dy = rk.DeviceBuffer.from_array(x.view(np.uint16)), rk.DeviceBuffer(m * n * 4)
+    prods = []
+    for t in w:
+        assert lib.rk_matmul_f16_dev(int(rk.pack(t)), dx.ptr, m, k, dy.ptr, None) == 0, lib.rk_last_error()
+        rk.synchronize()
+        prods.append(dy.download((m, n), np.uint16).view(np.float16))
+        ref = x.astype(np.float64) @ t.astype(np.float16).astype(np.float64).T
+        # f32 sums of K products (1e-5 of the largest, as in the few-tile tests), then one fp16 rounding
+        assert (np.abs(prods[-1] - ref) <= 1e-5 * np.abs(ref).max() + 2.0 ** -11 * np.abs(ref)).all()
+    wid = rk.pack_f16_glu(*w)
+    for kind, glue in ((rk.GLU_SILU, rk.silu_mul), (rk.GLU_GELU, rk.gelu_mul)):
+        want = glue(*[p.astype(np.float32) for p in prods])
+        for f16 in (0, 1):
+            assert lib.rk_matmul_f16_glu_dev(int(wid), dx.ptr, m, k, kind, dy.ptr, f16, None) == 0
+            rk.synchronize()
+            if f16:  # (the glue op on fp16 operands computes in f32 and rounds once)
+                assert (dy.download((m, n), np.uint16) == glue(*prods).view(np.uint16)).all()
+            else:
+                assert (dy.download((m, n), np.float32) == want).all()
