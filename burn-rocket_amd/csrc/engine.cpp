@@ -822,10 +822,11 @@ int launch_i8(const Weight &w, const int8_t *a, const float *as, int as_stride, 
 
 // One fp16 GEMM launch (glu: the gate|up epilogue form) with its split-K
 // workspace from the call's scratch: partial tiles, and arrival counters
-// zeroed when first allocated (every launch leaves them at zero).
+// zeroed when first allocated (every launch leaves them at zero). m_call: the
+// rows of the whole call, whose chunks of rows all sum K in the same order.
 int gemm_f16_run(CallScope &cs, const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k,
-                 const char *op, int glu = 0, int64_t n_out = 0, bool out_f16 = true) {
-  const int n1 = (int)(glu ? n_out : n), kwaves = rk_gemm_f16_kwaves((int)m, n1, (int)k, g_eng->num_cus);
+                 const char *op, int64_t m_call, int glu = 0, int64_t n_out = 0, bool out_f16 = true) {
+  const int n1 = (int)(glu ? n_out : n), kwaves = rk_gemm_f16_kwaves((int)m_call, n1, (int)k, g_eng->num_cus);
   if (rk_gemm_f16_skinny(kwaves, (int)m, n1, (int)k, glu != 0, g_eng->num_cus)) {
     HIP_TRY(rk_launch_gemm_f16_skinny(a, b, c, (int)m, (int)n, (int)k, glu, (int)n_out, out_f16, g_eng->num_cus, cs.st),
             op);
@@ -885,7 +886,7 @@ extern "C" int rk_matmul(rk_weight_id id, const float *x, int64_t m, int64_t k, 
     compute = [=, &cs](int64_t r0, int64_t r1) {
       const int64_t rows = r1 - r0;
       HIP_TRY(rk_launch_f32_to_f16(x32 + r0 * k, a16 + r0 * k, rows * k, st), "rk_matmul");
-      RK_TRY(gemm_f16_run(cs, a16 + r0 * k, w->codes, c16 + r0 * n, rows, n, k, "rk_matmul_fp16"));
+      RK_TRY(gemm_f16_run(cs, a16 + r0 * k, w->codes, c16 + r0 * n, rows, n, k, "rk_matmul_fp16", m));
       HIP_TRY(rk_launch_f16_to_f32(c16 + r0 * n, y32 + r0 * n, rows * n, st), "rk_matmul");
       return RK_OK;
     };
@@ -945,7 +946,7 @@ extern "C" int rk_matmul_f16(rk_weight_id id, const uint16_t *a, int64_t m, int6
   RK_TRY(scratch(cs, "mm_a16", (size_t)m * k * 2, (void **)&a16));
   RK_TRY(scratch(cs, "mm_c16", (size_t)m * n * 2, (void **)&c16));
   auto compute = [&](int64_t r0, int64_t r1) {
-    RK_TRY(gemm_f16_run(cs, a16 + r0 * k, w->codes, c16 + r0 * n, r1 - r0, n, k, "rocket_matmul_fp16"));
+    RK_TRY(gemm_f16_run(cs, a16 + r0 * k, w->codes, c16 + r0 * n, r1 - r0, n, k, "rocket_matmul_fp16", m));
     return RK_OK;
   };
   RK_TRY(staged(cs, {{a, nullptr, a16, (size_t)k * 2, 0}}, {{nullptr, c, c16, (size_t)n * 2, 0}}, m,
@@ -1043,7 +1044,7 @@ extern "C" int rk_matmul_f16_dev(rk_weight_id id, const void *a, int64_t m, int6
     return fail(RK_E_UNSUPPORTED, "rk_matmul_f16_dev", "gate|up weight: use rk_matmul_f16_glu_dev");
   if (m == 0) return RK_OK;  // an empty batch: nothing to compute (the reference returns [.., 0, N])
   CallScope cs(pick(stream));
-  RK_TRY(gemm_f16_run(cs, a, w->codes, c, m, w->n, k, "rk_matmul_f16_dev"));
+  RK_TRY(gemm_f16_run(cs, a, w->codes, c, m, w->n, k, "rk_matmul_f16_dev", m));
   g_eng->calls++;
   return RK_OK;
 }
@@ -1060,7 +1061,7 @@ extern "C" int rk_matmul_f16_glu_dev(rk_weight_id id, const void *a, int64_t m, 
   if (glu != RK_GLU_SILU && glu != RK_GLU_GELU) return fail(RK_E_SHAPE, op, "unknown glu kind");
   if (m == 0) return RK_OK;  // an empty batch: nothing to compute (the reference returns [.., 0, N])
   CallScope cs(pick(stream));
-  RK_TRY(gemm_f16_run(cs, a, w->codes, out, m, w->n, k, op, glu, w->glu_n, out_f16 != 0));
+  RK_TRY(gemm_f16_run(cs, a, w->codes, out, m, w->n, k, op, m, glu, w->glu_n, out_f16 != 0));
   g_eng->calls++;
   return RK_OK;
 }

@@ -127,3 +127,21 @@ def test_fp16_gate_up_equals_products_then_glue(rk, orc, m, k, n):
                 assert (dy.download((m, n), np.uint16) == glue(*prods).view(np.uint16)).all()
             else:
                 assert (dy.download((m, n), np.float32) == want).all()
+
+
+# Calls whose rows move in chunks: a short last chunk (688 + 12 rows, 1376 + 24), and chunks that by
+# themselves would split K over eight waves where the whole call splits it over four.
+@pytest.mark.parametrize("m,k,n", [(700, 1024, 3072), (1400, 1024, 3072), (9000, 768, 32)])
+def test_fp16_rows_of_a_host_call_follow_one_order(rk, m, k, n):
+    note(f"fp16 host call m={m} k={k} n={n}")
+    lib, r = rk.lib(), np.random.default_rng(m + n)
+    x = r.standard_normal((m, k)).astype(np.float16)
+    wid = rk.pack((r.standard_normal((n, k)) * 0.05).astype(np.float32))
+    dx, dy = rk.DeviceBuffer.from_array(x.view(np.uint16)), rk.DeviceBuffer(m * n * 2)
+    assert lib.rk_matmul_f16_dev(int(wid), dx.ptr, m, k, dy.ptr, None) == 0, lib.rk_last_error()
+    rk.synchronize()
+    want = dy.download((m, n), np.uint16).view(np.float16)
+    assert (rk.matmul(x.astype(np.float32), wid) == want.astype(np.float32)).all()
+    c = np.empty((m, n), np.float16)
+    assert lib.rk_matmul_f16(int(wid), x.ctypes.data, m, k, c.ctypes.data) == 0, lib.rk_last_error()
+    assert (c == want).all()
