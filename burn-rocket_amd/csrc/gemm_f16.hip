@@ -510,9 +510,9 @@ constexpr int CFG_KW8 = 100, CFG_KW4 = 101, CFG_KW8_64x32 = 102, CFG_KW8_32x64 =
               CFG_KW4_64x64 = 105;
 int kwaves_cfg(int kwaves, int M, int N, int K, bool glu, int num_cus) {
   const int64_t n32 = (N + 31) / 32, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
-  if (!glu || (kwaves == 8 ? m32 : m64) * n32 <= num_cus) return kwaves == 8 ? CFG_KW8 : CFG_KW4;
-  if (kwaves == 8) return m64 * n32 <= num_cus ? CFG_KW8_64x32 : CFG_KW8_32x64;
-  return K < 1536 ? CFG_KW4_SHORT : CFG_KW4_64x64;
+  if (!glu) return kwaves == 8 ? CFG_KW8 : CFG_KW4;
+  if (kwaves == 4) return K < 1536 ? CFG_KW4_SHORT : CFG_KW4_64x64;  // (more than one round at any size)
+  return m32 * n32 <= num_cus ? CFG_KW8 : m64 * n32 <= num_cus ? CFG_KW8_64x32 : CFG_KW8_32x64;
 }
 
 hipError_t launch_cfg(int c, const f16 *a, const f16 *b, f16 *d, int M, int N, int K, int ks, float *part,
@@ -649,7 +649,6 @@ hipError_t launch_glu_cfg(int c, const f16 *a, const f16 *b, void *d, int M, int
                           float *part, unsigned *cnt, hipStream_t st) {
   switch (c) {
     case CFG_KW8: return launch_kwaves<32, 32, 8, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
-    case CFG_KW4: return launch_kwaves<64, 32, 4, 3, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case CFG_KW8_64x32: return launch_kwaves<64, 32, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case CFG_KW8_32x64: return launch_kwaves<32, 64, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case CFG_KW4_SHORT: return launch_kwaves<64, 32, 4, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
