@@ -13,6 +13,14 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU")
 
 
+@pytest.fixture(params=["few-rows", "128-rows"])
+def attn_route(request, monkeypatch):
+    """Shapes of few query rows on the kernel the library picks for them, and on the 128-row kernel
+    (with its transposed V) that larger ones take."""
+    if request.param == "128-rows":
+        monkeypatch.setenv("RK_ATTN_FEW", "0")
+
+
 @pytest.fixture(scope="session")
 def orc():
     import oracle

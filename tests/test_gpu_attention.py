@@ -87,6 +87,7 @@ def test_config5_gqa_32_4_full(rk, orc):
     check_rows(orc, got, q, k, v, h, kv, d, d ** -0.5, _slices(s, 64), mode=1)
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("d", [32, 48, 64, 72, 80, 96, 112, 128, 256])
 @pytest.mark.parametrize("h,kv", [(4, 4), (8, 2), (16, 2), (6, 3)])
 def test_head_dims_and_groups(rk, orc, d, h, kv):
@@ -147,6 +148,7 @@ def test_mixed_slot_equals_separate_slots(rk, orc, d, rows, split, monkeypatch):
         check(orc, outs[0], orc.attention_ref(q, k, v, h, kv, d, d ** -0.5, 0.0, mode, window))
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("mode,window,n_q,n_kv,q0,k0", [
     (2, 17, 200, 200, 0, 0),      # band
     (3, 33, 200, 200, 0, 0),      # causal sliding window
@@ -219,6 +221,7 @@ def test_key_split_of_the_longest_causal_tiles(rk, orc, monkeypatch, forced, mod
                window=window, ref64=False)
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("mode,window,softcap,q0,k0,n_q,n_kv", [
     (2, 512, 0.0, 0, 0, 1200, 1200),       # sliding layer, one chunk
     (0, -1, 0.0, 0, 0, 700, 700),          # full layer
@@ -260,6 +263,7 @@ def test_gemma_attention_at_the_bench_size(rk, orc, mode, window):
     check_rows(orc, got, q, k, v, h, kv, d, d ** -0.5, _slices(s, 48), mode=mode, window=window)
 
 
+@pytest.mark.usefixtures("attn_route")
 def test_softcap(rk, orc):
     note("softcap 20")
     r = np.random.default_rng(99)
@@ -358,6 +362,7 @@ def test_flash_attn_head_dims_of_the_reference_contract(rk, orc, hd, dv):
         check(orc, got, ref)
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("d", [160, 192, 224])
 def test_token_major_head_dims_run_padded(rk, orc, d):
     """rk_attention_dev and rk_attention take the head dims of the reference's
@@ -409,6 +414,7 @@ def test_attention_is_deterministic(rk, orc):
     check(orc, a, orc.attention_flex(q, k, v, h, kv, d, d ** -0.5, 0.0, 1))
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("mode", [0, 1])
 def test_head_padding_invariance(rk, orc, mode):
     """Zero-padding the head dim 72 → 80 / 96 (the reference's padded-layout test,

@@ -41,18 +41,20 @@ def test_quantize_groups_is_bit_exact(rk, orc, m, group):
         assert (got[:, :-group] == q[:, :-group]).all()
 
 
-# Tiles of 128x64 and 64x64 at their edges, one group, an odd number of groups
-# (64: a stage that holds one group), columns and rows that end inside a tile,
-# and the size at which the tiles change.
-SHAPES = [(1, 128, 1), (63, 192, 65), (65, 384, 200), (129, 1152, 1000), (2050, 256, 1090)]
+# The pipelined kernel: its 64x64 tiles at their edges, one group, an odd number of groups (64: a
+# stage that holds one group), columns and rows that end inside a tile (those of few tiles only reach it
+# with RK_SKINNY=0; as they are they run on the few-tile kernels), and its 128x64 tiles with two stages and
+# with ten, more than its ring of three holds, of which the last is half filled (group 64).
+SHAPES = [(1, 128, 1), (63, 192, 65), (65, 384, 200), (129, 1152, 1000), (2050, 256, 1090), (2050, 1216, 1090)]
 
 
 @pytest.mark.parametrize("group", [64, 128])
-@pytest.mark.parametrize("m,k,n", SHAPES)
-def test_group_gemm(rk, orc, m, k, n, group):
+@pytest.mark.parametrize("m,k,n,skinny", [(*s, v) for s in SHAPES for v in ("1", "0") if v == "1" or s[0] < 2000])
+def test_group_gemm(rk, orc, monkeypatch, m, k, n, skinny, group):
+    monkeypatch.setenv("RK_SKINNY", skinny)
     if k % group:
         k += group - k % group
-    note(f"group gemm m={m} k={k} n={n} group={group}")
+    note(f"group gemm m={m} k={k} n={n} group={group} RK_SKINNY={skinny}")
     r = np.random.default_rng(m + k + n + group)
     x = r.standard_normal((m, k)).astype(np.float32)
     w = (r.standard_normal((n, k)) * 0.02).astype(np.float32)

@@ -411,6 +411,7 @@ def _attn_packed(rk, q, k, v, hq, hk, d, mode, n):
         dev.free()
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("d,hq,hk,mode", [(128, 4, 2, 1), (72, 3, 3, 0), (64, 8, 1, 1)])
 def test_attention_strided_on_a_qkv_buffer(rk, d, hq, hk, mode):
     n = 301
@@ -451,6 +452,7 @@ def test_qk_norm_rope_row_groups(rk, orc, groups, monkeypatch):
     assert (got == qknr_ref(orc, x, hq, hk, d, wq, wk, c, sn, "f16")).all()
 
 
+@pytest.mark.usefixtures("attn_route")
 def test_qwen3_attention_chain_in_place(rk, orc):
     """qkv GEMM into one buffer → q/k norm + RoPE in place → attention reading q, k, v where
     they lie; against the same ops on separate tensors (bit for bit) and the oracle."""
@@ -516,6 +518,7 @@ def test_qk_norm_rope_head_counts(rk, orc, hq, hk, s):
         assert (got == qknr_ref(orc, x, hq, hk, d, wq, wk, c, sn, dt)).all()
 
 
+@pytest.mark.usefixtures("attn_route")
 @pytest.mark.parametrize("s,hq,hk,d,mode", [(203, 4, 2, 128, 1), (150, 3, 3, 72, 0), (64, 8, 1, 64, 1),
                                             (1, 2, 1, 128, 1), (300, 3, 1, 256, 0), (300, 3, 1, 256, 1)])
 def test_attention_qkv_equals_prologue_then_strided_attention(rk, orc, s, hq, hk, d, mode):

@@ -7,9 +7,11 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# M, K, N: one row, the 32-row tile edges, K of one block / less than one stage
-# per wave / ends inside a stage / more than two stages per wave.
-SHAPES = [(1, 32, 1), (16, 160, 40), (33, 1152, 33), (32, 416, 200), (5, 3072, 96), (95, 4128, 65)]
+# M, K, N: one row, the 16-row tile edges, K of one block / less than one stage
+# per wave / ends inside a stage / more than two stages per wave; and more tiles
+# than one round of workgroups, ragged both ways (the last, 16-row tiles walked by
+# one wave each).
+SHAPES = [(1, 32, 1), (16, 160, 40), (33, 1152, 33), (32, 416, 200), (5, 3072, 96), (95, 4128, 65), (100, 416, 3001)]
 
 
 def note(msg):
@@ -69,11 +71,12 @@ def test_skinny_f16(rk, orc, m, k, n):
           (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32), True)
 
 
-# K split over the waves of 32x32 tiles (8 waves) and 64x32 tiles (4 waves): one
-# row, tile edges, K of less than two stages per wave and one that ends inside
-# a stage, odd N, and the largest grids of either tile.
+# K split over the waves of 32x32 tiles (8 waves) and 64x32 tiles (4 waves, the last
+# three): one row, tile edges, K of less than two stages per wave and one that ends
+# inside a stage, odd N, and the largest grids of either tile. (33 rows of K = 768
+# run on the 16-row tiles.)
 @pytest.mark.parametrize("m,k,n", [(9, 1536, 1), (33, 768, 1050), (64, 1544, 3000), (255, 776, 1000), (300, 1160, 800),
-                                   (512, 3072, 1024), (65, 4304, 2001)])
+                                   (65, 4304, 2001), (70, 776, 3001), (450, 1160, 1000), (512, 3072, 1024)])
 def test_kwaves_f16(rk, orc, m, k, n):
     note(f"fp16 K over waves m={m} k={k} n={n}")
     r = np.random.default_rng(m + k + n)
@@ -91,7 +94,8 @@ def test_kwaves_f16(rk, orc, m, k, n):
 
 @pytest.mark.parametrize("glu", ["silu", "gelu"])
 @pytest.mark.parametrize("f16", [False, True])
-@pytest.mark.parametrize("m,k,n", [(9, 1536, 5), (40, 776, 1900), (64, 1160, 1900), (130, 3072, 300)])
+@pytest.mark.parametrize("m,k,n", [(9, 1536, 5), (40, 776, 1900), (64, 1160, 1900), (130, 3072, 300), (100, 1160, 1900),
+                                   (20, 1160, 4300), (70, 776, 3001), (450, 1600, 1000)])
 def test_kwaves_f16_glu(rk, orc, m, k, n, glu, f16):
     """gate|up against the glue of float64 products rounded to fp16: a product next to a rounding
     midpoint may round the other way (one fp16 step of the gate or up value)."""
@@ -116,7 +120,8 @@ def test_kwaves_f16_glu(rk, orc, m, k, n, glu, f16):
 @pytest.mark.parametrize("m,k,n", [(1, 64, 3), (8, 1152, 40), (32, 416, 64), (29, 3072, 17),
                                    (24, 128, 1500), (128, 256, 72), (9, 96, 4000)])
 def test_skinny_glu_equals_products_then_glue(rk, orc, m, k, n, glu):
-    """The fused forms give what the two plain products and the glue op give, bit for bit."""
+    """The fused forms give what the two plain products and the glue op give, bit for bit (larger
+    shapes: test_gpu_sum_order.py)."""
     note(f"skinny gate|up m={m} k={k} n={n} {glu}")
     lib, r = rk.lib(), np.random.default_rng(m + k + n)
     kind, glue = (rk.GLU_SILU, rk.silu_mul) if glu == "silu" else (rk.GLU_GELU, rk.gelu_mul)

@@ -351,11 +351,15 @@ def test_q8_0_blocks_split_on_the_device_keep_every_scale_exactly(rk, orc):
 # Fused gate|up GEMM with the MLP glue in the epilogue: glue(gate·x, up·x)
 # against the oracle's two W8A8 products and its glue (host.rs:12-39).
 # Shapes select each tile configuration of the fused launch on a 256-CU
-# MI355X: 2 / 224 / 256 tiles of 128x128 over the interleaved rows (n = 100
-# also leaves padding rows in the last 16-row group).
+# MI355X: few tiles; 128x64 tiles, from 2 tiles of 128x128 over the interleaved
+# rows (70 rows, which come here with RK_SKINNY=0 only; n = 100 also leaves padding
+# rows in the last 16-row group) and from 128 (ragged rows and outputs); 224 and
+# 256 tiles of 128x128.
 @pytest.mark.parametrize("glu", ["silu", "gelu"])
-@pytest.mark.parametrize("m,k,n", [(70, 512, 100), (1700, 256, 1024), (2048, 256, 1024)])
-def test_w8a8_glu_fused(rk, orc, glu, m, k, n):
+@pytest.mark.parametrize("m,k,n,skinny", [(70, 512, 100, "1"), (70, 512, 100, "0"), (1001, 416, 1000, "1"),
+                                          (1700, 256, 1024, "1"), (2048, 256, 1024, "1")])
+def test_w8a8_glu_fused(rk, orc, monkeypatch, glu, m, k, n, skinny):
+    monkeypatch.setenv("RK_SKINNY", skinny)
     r = np.random.default_rng(m + k + n + len(glu))
     x = r.standard_normal((m, k)).astype(np.float32)
     gate = (r.standard_normal((n, k)) * 0.05).astype(np.float32)
@@ -376,7 +380,7 @@ def test_w8a8_glu_fused(rk, orc, glu, m, k, n):
         else:
             wid = rk.pack_q8_0_glu_f32(gate, up)
         for f16out in (False, True):
-            note(f"W8A8 fused {glu} m={m} k={k} n={n} packer={packer} f16out={f16out}")
+            note(f"W8A8 fused {glu} m={m} k={k} n={n} packer={packer} f16out={f16out} RK_SKINNY={skinny}")
             dc = rk.DeviceBuffer(m * n * (2 if f16out else 4))
             rc = lib.rk_matmul_w8a8_glu_dev(int(wid), dq.ptr, ds.ptr, m, k, kind, dc.ptr, int(f16out), None)
             assert rc == 0, lib.rk_last_error()
