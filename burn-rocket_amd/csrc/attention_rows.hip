@@ -5,9 +5,9 @@
 // keys between barriers, with V transposed by a launch of its own first. With a
 // few rows that is one long serial walk on a handful of CUs: what bounds the
 // call is its latency. Here a workgroup takes up to 16·RT rows of one kv head
-// (row r ↔ query r / G, head r % G of the group) and one of S key ranges; its
-// four waves walk the range's 32-key chunks on their own (wave w chunks w,
-// w + 4, ...), with no barrier until their softmax states meet in LDS. With
+// (row r ↔ query r / G, head r % G of the group) and one of S key ranges; its RW
+// waves (8; 4 for head dim 256) walk the range's 32-key chunks on their own (wave
+// w chunks w, w + RW, ...), with no barrier until their softmax states meet in LDS. With
 // S > 1 the states then meet in a workspace: the workgroup that arrives last
 // merges all S, in split order whichever it is, and nothing waits on another.
 //
