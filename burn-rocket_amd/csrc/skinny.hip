@@ -38,7 +38,11 @@ namespace {
 template <bool GROUPED, int GB, int TN>
 struct SkinnyI8Geom {
   static constexpr int PB = TN == 1 ? 2 : 1;  // product buffers: two save a barrier per round
-  static constexpr int SLOT = (1 + TN) * 2048;                   // a stage's codes: 16 rows, 16·TN columns
+  // Codes of 16 rows or columns, and 64 bytes that keep the compiler from pairing
+  // the reads of two tiles in one instruction: on the same banks, the pair would
+  // take twice its time.
+  static constexpr int TILE = 2048 + 64;
+  static constexpr int SLOT = (1 + TN) * TILE;                   // a stage's codes: 16 rows, 16·TN columns
   static constexpr int SC = TN * 256 + (GROUPED ? 256 : 0);      // its scales, [column][4], [row][4]
   static constexpr int NS = 3;  // scale slots: a round's are folded while the next one's land
   // an element's products of a round, and 16 bytes that spread them over the banks
@@ -51,8 +55,9 @@ struct SkinnyI8Geom {
 template <bool GROUPED>
 struct WaveI8Geom {
   static constexpr int ST = 2;
-  // a stage: rows [16][128], columns, column scales [16][4], row scales [group][16]
-  static constexpr int W_OFF = 2048, WS_OFF = 4096, AS_OFF = WS_OFF + 256;
+  // a stage: rows [16][128], column scales [16][4], columns (apart from the rows, as
+  // above), row scales [group][16]
+  static constexpr int WS_OFF = 2048, W_OFF = WS_OFF + 256, AS_OFF = W_OFF + 2048;
   static constexpr int SLOT = AS_OFF + (GROUPED ? 256 : 0);
   static constexpr int SMEM = 4 * ST * SLOT;
 };
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(SNW * 64, 2) void skinny_i8_kernel(
 #pragma unroll
     for (int q = 0; q < 2; ++q) bdma16(ra, slot + q * 1024, v[q], k0);
 #pragma unroll
-    for (int q = 0; q < 2 * TN; ++q) bdma16(rw, slot + 2048 + q * 1024, v[q & 1], (q >> 1) * 16 * K + k0);
+    for (int q = 0; q < 2 * TN; ++q) bdma16(rw, slot + (1 + (q >> 1)) * G::TILE + (q & 1) * 1024, v[q & 1], (q >> 1) * 16 * K + k0);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_PTR(sc + j * 256), 4, v_ws,
@@ -130,7 +135,7 @@ __global__ __launch_bounds__(SNW * 64, 2) void skinny_i8_kernel(
     for (int b = 0; b < 4; ++b) {
       a[b] = *(const long *)(slot + f_off[b]);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) w[j][b] = *(const long *)(slot + (1 + j) * 2048 + f_off[b]);
+      for (int j = 0; j < TN; ++j) w[j][b] = *(const long *)(slot + (1 + j) * G::TILE + f_off[b]);
     }
     WAIT_LGKMCNT0();  // the slot is read: refilled while the products are formed
     asm volatile("" ::: "memory");
@@ -251,8 +256,11 @@ static hipError_t launch_skinny_i8_tn(const I8GemmArgs &g, hipStream_t st) {
 // with more tiles than one round of the kernel above there are waves enough to
 // hide a stage's issue and latency, and handing the products on costs more. A
 // workgroup is 2x2 such waves (what they read in common hits the CU's cache),
-// each with an LDS ring of two stages of its own. While a stage's products are
-// formed the next one is read and its slot refilled; then the stage is folded.
+// each with an LDS ring of two stages of its own (three to six are slower). While
+// a stage's products are formed the next one is read and its slot refilled; then
+// the stage is folded. Every wave copies its own operands: four waves ask a CU's
+// cache for 17 KB a stage, 272 clocks of its 64 bytes per clock, of about 420 that
+// a stage takes.
 // gate|up: the left waves have gate, the right ones up.
 template <bool GROUPED, bool WSF16, int GB, int GLU, bool OUT_F16>
 __global__ __launch_bounds__(256, 2) void wave_i8_kernel(
