@@ -54,8 +54,10 @@ constexpr int ROWB = 128;  // bytes per LDS row of one stage
 // glue runs in f32, and C is [M, n_out] f32 (OUT_F16: fp16).
 // SPLIT = false is the unsplit kernel (ksplit must be 1): the partial
 // exchange is compiled out, and with it the registers it holds.
+// SETS > 1: stage s adds to accumulator set s mod SETS and the sets are added at
+// the end, the sums of gemm_f16_kwaves_kernel on SETS waves in this kernel's time.
 template <int BM, int BN, int WM, int WN, int ST, int MINW, int GLU = 0, bool OUT_F16 = true,
-          bool SPLIT = false>
+          bool SPLIT = false, int SETS = 1>
 __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
     const f16 *__restrict__ A, const f16 *__restrict__ B, void *__restrict__ Cv, int M, int N, int K,
     int tiles_m, int tiles_n, int group_m, int n_out, int ksplit, float *__restrict__ part,
@@ -74,6 +76,7 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
   constexpr int L = (A_INS + B_INS) / NW;
   static_assert(TM * 16 * WM == BM && TN * 16 * WN == BN, "mfma split");
   static_assert(ST >= 2 && (ST - 1) * L <= 63, "pipeline depth");
+  static_assert(SETS == 1 || !SPLIT, "one split of K");
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -141,18 +144,21 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
     for (int j = 0; j < TN; ++j) fb[BUF][j] = *(const half8 *)(base + b_row + fch + j * 16 * ROWB);
   };
 
-  floatx4 acc[TM][TN];
+  floatx4 sets[SETS][TM][TN];
+  auto &acc = sets[0];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int z = 0; z < SETS; ++z)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) sets[z][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   constexpr int T = TM * TN;
-  auto mfmas = [&](auto buf_c) {
-    constexpr int BUF = decltype(buf_c)::value;
+  auto mfmas = [&](auto set_c, auto buf_c) {
+    constexpr int Z = decltype(set_c)::value, BUF = decltype(buf_c)::value;
     static_for<T>([&](auto u_c) {
       constexpr int U = decltype(u_c)::value, I = U / TN, J = U % TN;
-      acc[I][J] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[BUF][J], fa[BUF][I], acc[I][J], 0, 0, 0);
+      sets[Z][I][J] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[BUF][J], fa[BUF][I], sets[Z][I][J], 0, 0, 0);
     });
   };
   // One MFMA, one copy; one MFMA, one fragment read; then the rest.
@@ -178,10 +184,10 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
   BARRIER();
   load_frags(ic<0>{}, 0, fch0);
 
-  for (int s = 0; s < KT; ++s) {
+  auto stage = [&](auto set_c, int s) __attribute__((always_inline)) {
     // Sub-step 0 (register set 0) while sub-step 1's fragments are read.
     load_frags(ic<1>{}, s, fch1);
-    mfmas(ic<0>{});
+    mfmas(set_c, ic<0>{});
     interleave(ic<0>{});
     __builtin_amdgcn_sched_barrier(0);
     // Stage s+1 visible to all waves (stages up to s+ST-1 were issued), and
@@ -194,11 +200,22 @@ __global__ __launch_bounds__(WM *WN * 64, MINW) void gemm_f16_kernel(
     BARRIER();
     issue(s + ST);
     load_frags(ic<0>{}, s + 1, fch0);
-    mfmas(ic<1>{});
+    mfmas(set_c, ic<1>{});
     interleave(ic<L>{});
     __builtin_amdgcn_sched_barrier(0);
-  }
+  };
+  for (int s = 0; s < KT; s += SETS)
+    static_for<SETS>([&](auto z_c) __attribute__((always_inline)) {
+      constexpr int Z = decltype(z_c)::value;
+      if (Z == 0 || s + Z < KT) stage(z_c, s + Z);
+    });
   WAIT_VMCNT(0);  // no copy may still be writing LDS when the workgroup ends
+#pragma unroll
+  for (int z = 1; z < SETS; ++z)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += sets[z][i][j];
 
   if constexpr (SPLIT) {
     // Partial slot of split j: [wave][tile u][lane] 16-byte entries.
@@ -454,13 +471,14 @@ static hipError_t launch_kwaves(const f16 *A, const f16 *B, void *C, int M, int 
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int ST, int MINW, int GLU = 0, bool OUT_F16 = true>
+template <int BM, int BN, int WM, int WN, int ST, int MINW, int GLU = 0, bool OUT_F16 = true, int SETS = 1>
 static hipError_t launch_gemm_f16(const f16 *A, const f16 *B, void *C, int M, int N, int K,
                                   int ksplit, float *part, unsigned *cnt, hipStream_t st, int n_out = 0) {
   constexpr int smem = ST * (BM + BN) * ROWB;
   static_assert(smem <= 160 * 1024, "LDS per workgroup");
-  auto kern = ksplit > 1 ? gemm_f16_kernel<BM, BN, WM, WN, ST, MINW, GLU, OUT_F16, true>
-                         : gemm_f16_kernel<BM, BN, WM, WN, ST, MINW, GLU, OUT_F16, false>;
+  auto kern = gemm_f16_kernel<BM, BN, WM, WN, ST, MINW, GLU, OUT_F16, false, SETS>;
+  if constexpr (SETS == 1)
+    if (ksplit > 1) kern = gemm_f16_kernel<BM, BN, WM, WN, ST, MINW, GLU, OUT_F16, true>;
   static bool attr_set[2] = {false, false};
   if (!attr_set[ksplit > 1]) {
     hipError_t e = hipFuncSetAttribute((const void *)kern,
@@ -500,18 +518,19 @@ constexpr F16Cfg F16_CFGS[] = {
 constexpr int N_F16_CFGS = sizeof(F16_CFGS) / sizeof(F16_CFGS[0]);
 // Configurations of gemm_f16_kwaves_kernel, by the waves K is split over: 32x32
 // tiles on 8, 64x32 on 4, one per CU. A gate|up product has twice the tiles of the
-// plain product whose split it takes: where those are more than one round, larger
-// tiles with fewer stages in flight, or for a short K on 4 waves several
-// workgroups per CU (MI355X, us: 8 waves, 1024->2x1024 256 rows 64x32 tiles 5.5,
-// 32x32 two per CU 6.1; 3072->2x1024 200 rows 64x32 8.7, 32x64 11.8; 4 waves,
-// 1024->2x3072 128 rows 64x32 6.7, 64x64 7.5; 2048->2x1024 512 rows 64x64 10.1,
-// 64x32 11.2).
-constexpr int CFG_KW8 = 100, CFG_KW4 = 101, CFG_KW8_64x32 = 102, CFG_KW8_32x64 = 103, CFG_KW4_SHORT = 104,
-              CFG_KW4_64x64 = 105;
+// plain product whose split it takes: where those are more than one round, on 8
+// waves larger tiles with fewer stages in flight (MI355X, us: 1024->2x1024 256
+// rows 64x32 tiles 5.5, 32x32 two per CU 6.1; 3072->2x1024 200 rows 64x32 8.7, 32x64
+// 11.8). Instead of 4 waves, gemm_f16_kernel with four accumulator sets on 64x64
+// tiles of eight waves, at most one per CU (us, there and unsplit: 1024->2x1024 512
+// rows 5.9 and 6.3, 2048->2x768 640 rows 9.0 and 9.1, 4304->2x1536 161 rows 19.7 and
+// 20.1; K over 4 waves on 64x32 or 64x64 tiles 6.8, 10.4 and 17.7; sets on four
+// waves, 128x64 tiles or a deeper ring: slower).
+constexpr int CFG_KW8 = 100, CFG_KW4 = 101, CFG_KW8_64x32 = 102, CFG_KW8_32x64 = 103, CFG_SETS4 = 104;
 int kwaves_cfg(int kwaves, int M, int N, int K, bool glu, int num_cus) {
   const int64_t n32 = (N + 31) / 32, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
   if (!glu) return kwaves == 8 ? CFG_KW8 : CFG_KW4;
-  if (kwaves == 4) return K < 1536 ? CFG_KW4_SHORT : CFG_KW4_64x64;  // (more than one round at any size)
+  if (kwaves == 4) return CFG_SETS4;
   return m32 * n32 <= num_cus ? CFG_KW8 : m64 * n32 <= num_cus ? CFG_KW8_64x32 : CFG_KW8_32x64;
 }
 
@@ -587,8 +606,7 @@ double cfg_time(int c, int ks, int M, int N, int K, int num_cus) {
 // tiles of a plain product are slower (3072->1024, 512 rows: 12.1 and 10.5 us on 4
 // and 8 waves). The fused form takes the plain one's split although it has twice
 // the tiles: with a split of its own it would differ from the plain products by
-// their rounding. At the upper end that costs a tenth (1024->2x1024 512 rows 6.4 us
-// unsplit, 6.9 on four waves; 2048->2x1024 9.2 and 10.1).
+// their rounding.
 int rk_gemm_f16_kwaves(int M, int n, int K, int num_cus) {
   if (rk_knob("RK_F16_TILE", -1) >= 0 || rk_knob("RK_F16_KSPLIT", 1) != 1) return 1;
   const bool skinny = rk_knob("RK_SKINNY", 1) != 0;
@@ -651,8 +669,8 @@ hipError_t launch_glu_cfg(int c, const f16 *a, const f16 *b, void *d, int M, int
     case CFG_KW8: return launch_kwaves<32, 32, 8, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case CFG_KW8_64x32: return launch_kwaves<64, 32, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
     case CFG_KW8_32x64: return launch_kwaves<32, 64, 8, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
-    case CFG_KW4_SHORT: return launch_kwaves<64, 32, 4, 1, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
-    case CFG_KW4_64x64: return launch_kwaves<64, 64, 4, 2, GLU, OUT_F16>(a, b, d, M, N, K, st, n_out);
+    case CFG_SETS4:
+      return launch_gemm_f16<64, 64, 4, 2, 4, 1, GLU, OUT_F16, 4>(a, b, d, M, N, K, 1, nullptr, nullptr, st, n_out);
     case 0: return launch_gemm_f16<256, 128, 4, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 1: return launch_gemm_f16<192, 192, 2, 2, 3, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);
     case 2: return launch_gemm_f16<128, 128, 2, 2, 4, 2, GLU, OUT_F16>(a, b, d, M, N, K, ks, part, cnt, st, n_out);

@@ -99,11 +99,12 @@ def test_int8_gate_up_equals_products_then_glue(rk, orc, monkeypatch, m, k, n):
 
 
 # K below 768 in each tile the few-tile kernel has; from there one row tile, tiles as wide
-# as a plain product's and twice as wide, K over eight waves, over four and unsplit.
+# as a plain product's and twice as wide, K over eight waves, over four (the fused form with
+# four accumulator sets: 16, 13, 19, 25 and 14 stages, full and ragged tiles) and unsplit.
 @pytest.mark.parametrize("m,k,n", [(24, 128, 1500), (40, 96, 1500), (20, 192, 4200), (12, 136, 4300), (8, 1024, 3072),
                                    (33, 1024, 3072), (64, 1024, 3072), (128, 1024, 3072), (256, 776, 1000),
                                    (20, 1160, 4300), (100, 1160, 1900), (70, 776, 3001), (450, 1600, 1000),
-                                   (500, 1160, 1000), (300, 1024, 3072)])
+                                   (500, 1160, 1000), (257, 888, 1000), (300, 1024, 3072)])
 def test_fp16_gate_up_equals_products_then_glue(rk, orc, m, k, n):
     note(f"fp16 gate|up m={m} k={k} n={n}")
     lib, r = rk.lib(), np.random.default_rng(m + k + n)
