@@ -205,8 +205,9 @@ int rk_weight_info(rk_weight_id id, int *kind, int64_t *n, int64_t *k,
 
 /* y[M, N] = x[M, K] · Wᵀ for any resident weight, host f32 in and out
  * (`rocket_matmul` → matmul_impl, ext.rs:627, ext.rs:1208-1232):
- *   F16: x → fp16 (RNE), fp16 GEMM with f32 accumulation, fp16 result widened
- *        to f32 (matmul_f16, ext.rs:1437-1499);
+ *   F16: x → fp16 (RNE), fp16 GEMM with f32 accumulation (the order of the
+ *        sums as at rk_matmul_f16_dev), fp16 result widened to f32
+ *        (matmul_f16, ext.rs:1437-1499);
  *   I8 : x quantized per row per weight group (quantize_i8_rows, ext.rs:1017),
  *        C = Σ_g (a_s[m,g]·w_s[n,g])·P_g with exact int32 P_g (matmul_i8,
  *        ext.rs:1505; detile_accum_i8_scaled, layout.rs:504-540);
@@ -235,7 +236,15 @@ int rk_matmul_i8_gw(rk_weight_id id, const int8_t *a, const float *a_scale,
 int rk_matmul_i8(rk_weight_id id, const int8_t *a, int64_t m, int64_t k, int32_t *c);
 
 /* fp16 GEMM on device buffers: a fp16 [M, K], c fp16 [M, N]
- * (`RocketCtx::matmul_prepacked`, lib.rs:244-254). K % 8 == 0. */
+ * (`RocketCtx::matmul_prepacked`, lib.rs:244-254). K % 8 == 0.
+ *
+ * Order of the f32 sums, here and in every fp16 product: one sum over
+ * ascending K, or, for few outputs, eight or four partial sums over parts of K
+ * added at the end. Which of the three depends on M, N and K only and is
+ * the same for all rows and columns of a call, also where a host entry runs its
+ * rows in chunks. The same row in a call with another M can therefore
+ * differ by the rounding of the f32 sums, which moves an fp16 result next to a
+ * midpoint by one step. Calls of equal sizes give equal bits. */
 int rk_matmul_f16_dev(rk_weight_id id, const void *a, int64_t m, int64_t k,
                       void *c, rk_stream stream);
 
@@ -250,7 +259,9 @@ int rk_matmul_f16_dev(rk_weight_id id, const void *a, int64_t m, int64_t k,
  * the plain GEMM's output is, then the glue runs in f32 with no FMA
  * contraction. a fp16 [M, K]; out f32 or (out_f16) fp16 [M, n]. The weight
  * comes from rk_pack_f16_glu (f32 gate and up, each [n, K], rounded to fp16
- * and interleaved per 16 rows); such a weight is only accepted here. */
+ * and interleaved per 16 rows); such a weight is only accepted here. Either
+ * product sums K in the order of rk_matmul_f16_dev on its own [n, K] weight: the
+ * result is that of the two plain products and the glue, bit for bit. */
 int rk_pack_f16_glu(const float *gate, const float *up, int64_t n, int64_t k, rk_weight_id *id);
 int rk_matmul_f16_glu_dev(rk_weight_id id, const void *a, int64_t m, int64_t k, int glu, void *out,
                           int out_f16, rk_stream stream);
@@ -270,7 +281,8 @@ int rk_quantize_rows_dev(const float *x, int64_t m, int64_t k, int64_t group,
  * acc + fl(fl(a_s·w_s)·P_g): weights whose every scale is an fp16 value (GGUF
  * Q8_0 d) fold fma(fl(P_g·d), a_s, acc), others fma(P_g, fl(a_s·w_s), acc).
  * Both stay within 1e-5 of the largest output against the reference formula
- * at the config-2 shapes. rk_matmul_i8_gw folds every weight the second way. */
+ * at the config-2 shapes. rk_matmul_i8_gw folds every weight the second way.
+ * A row's result does not depend on M. */
 int rk_matmul_w8a8_dev(rk_weight_id id, const int8_t *a, const float *a_scale,
                        int64_t a_group, int64_t m, int64_t k, float *c,
                        rk_stream stream);
@@ -315,11 +327,16 @@ int rk_attention(const float *q, const float *k, const float *v, int64_t n_q,
                  float scale, float softcap, int mask_mode, int64_t window,
                  int64_t q0, int64_t k0, float *out);
 
-/* The same on fp16 device buffers in the token-major layout. Library scratch
- * holds V transposed and, when the launch has at most half as many query
- * tiles as the GPU has CUs, the partial softmax states of query tiles whose
- * keys are split between two workgroups (merged in a fixed order: results are
- * the same from call to call). */
+/* The same on fp16 device buffers in the token-major layout. With few query
+ * rows (decode, short chunks: at most two 16-row tiles per CU over all kv heads,
+ * half a tile for head dim 256) K and V are read where they lie and a tile's keys
+ * are split over the waves of up to 16 workgroups, whose partial softmax states go
+ * through library scratch. Otherwise library scratch holds V transposed and, when the
+ * launch has at most half as many query tiles as the GPU has CUs, or causal and at
+ * most one per CU, the partial states of query tiles whose keys are split between two
+ * workgroups. States are merged in a fixed order: results are the same from call
+ * to call. The split depends on the call's sizes, so a query row's result can
+ * differ in rounding between calls of different n_q. */
 int rk_attention_dev(const void *q, const void *k, const void *v, int64_t n_q,
                      int64_t n_kv, int n_head, int n_kv_heads, int head_dim,
                      float scale, float softcap, int mask_mode, int64_t window,
@@ -333,11 +350,13 @@ int rk_attention_dev(const void *q, const void *k, const void *v, int64_t n_q,
  * round_up(n_kv, 64) · 2 bytes with dv_pad = head_dim rounded up to 16, is
  * larger return RK_E_NOMEM. All calls on one GPU share that array and each
  * call rewrites it: calls whose work overlaps on the device (different streams
- * with no ordering between them) race and give wrong results. It never
- * splits a query tile's keys (that needs a workspace), and it refuses head
- * dims 160, 192 and 224 with RK_E_UNSUPPORTED (rk_attention_dev runs those
- * zero-padded to 256 in scratch); otherwise the same arguments and results as
- * rk_attention_dev (bit for bit when that split is off, RK_ATTN_SPLIT=1). */
+ * with no ordering between them) race and give wrong results. It always runs the
+ * transposed-V form and never splits a query tile's keys (that needs a
+ * workspace), and it refuses head dims 160, 192 and 224 with RK_E_UNSUPPORTED
+ * (rk_attention_dev runs those zero-padded to 256 in scratch); otherwise the same
+ * arguments as rk_attention_dev, and the same results within the rounding of
+ * the sums (bit for bit under RK_ATTN_SPLIT=1, which turns the few-row form and
+ * the split off). */
 #define RK_NOALLOC_SCRATCH_BYTES (32u << 20)
 int rk_attention_dev_noalloc(const void *q, const void *k, const void *v, int64_t n_q,
                              int64_t n_kv, int n_head, int n_kv_heads, int head_dim, float scale,
