@@ -394,7 +394,9 @@ struct RowsPlan {
 RowsPlan rows_plan(const AttnArgs &a) {
   const int G = a.n_head / a.n_kv_heads;
   const int64_t R = (int64_t)G * a.n_q;
-  int64_t keys = a.n_kv;  // that a row tile can see
+  // Keys that a row tile can see. Causal counts them all, also where q0 leaves the
+  // first queries fewer: their last ranges are empty then and merge with weight 0.
+  int64_t keys = a.n_kv;
   if (a.mask_mode == RK_MASK_WINDOW) keys = std::min<int64_t>(keys, 2 * std::min<int64_t>(a.window, keys) + a.n_q);
   if (a.mask_mode == RK_MASK_CAUSAL_WINDOW) keys = std::min<int64_t>(keys, std::min<int64_t>(a.window, keys) + a.n_q);
   const int64_t chunks = (std::max<int64_t>(keys, 1) + CK - 1) / CK;

@@ -224,9 +224,11 @@ __global__ __launch_bounds__(256) void quantize_tokens_kernel(const float *__res
 // Groups of 8·LPG values (32, 64, 128, 256 or 512; the group divides K): each
 // lane quantizes 8 consecutive values, so LPG neighbouring lanes hold one
 // group (groups never straddle a row) and the group maximum is log2(LPG) lane
-// swaps. Same arithmetic as above. HBM-bound: one read of x and one write of
-// the codes (2777x1024 in groups of 128, MI355X: 6.1 us; one workgroup per
-// row with LDS atomics, quantize_rows_kernel, takes 16.1 us).
+// swaps. Same arithmetic as above. One read of x, one write of the codes; one
+// thread has one trip to memory, so a launch of this size is its start and that
+// trip, not bandwidth (2777x1024 in groups of 128, MI355X: 6.1 us for 14 MB, 2.3
+// TB/s, half a large copy's rate, VALU 11 % busy; one workgroup per row with LDS
+// atomics, quantize_rows_kernel, takes 16.1 us).
 template <int LPG>
 __global__ __launch_bounds__(256) void quantize_groups_kernel(const float *__restrict__ x, int64_t n8,
                                                               int8_t *__restrict__ q,

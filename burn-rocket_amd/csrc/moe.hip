@@ -539,7 +539,8 @@ __global__ __launch_bounds__(NW * 64, 2) void moe_q8_kernel(
 // registers: NQ·8 rows fold NQ·4 of them. Few registers and little LDS keep
 // three workgroups on a CU, where the 128-row kernel's two left a second, nearly
 // empty round (30B-A3B experts, 8 tokens: 612 workgroups). HBM-bound on the
-// experts' weights. The planned call on that layer, MI355X, ring kernels -> here:
+// experts' weights (8 tokens: gate|up fetches 184 MB at 5.3 TB/s, down 93 MB at
+// 3.6; VALU at most 12 % busy). The planned call on that layer, MI355X, ring kernels -> here:
 // 1 token 38.4 -> 28.9 us, 8 tokens 78.2 -> 62.7 (4.4 TB/s), 64 tokens 152.9 ->
 // 137.5, 128 tokens 156.7 -> 145.0 (4.7 TB/s).
 template <bool GU, int NQ>
