@@ -6,7 +6,7 @@
 // a grid of a few dozen workgroups. Measured on MI355X (us per call, tiled
 // kernel -> here):
 //   int8 per token   12 rows, 1024->3072 8.7 -> 4.1;  3072->1024 19.8 -> 4.9;
-//                    256 rows, 1024->3072 9.3 -> 7.1; 3072->1024 20.5 -> 8.0
+//                    256 rows, 1024->3072 9.3 -> 7.0; 3072->1024 20.5 -> 7.9
 //   int8 group 32    12 rows, 1024->3072 11.2 -> 4.4; 256 rows, 3072->1024 28.5 -> 8.8
 //   fp16             1 row, 1024->3072 5.4 -> 3.4;    64 rows, 1024->1024 5.8 -> 3.9
 #include "common.hpp"
